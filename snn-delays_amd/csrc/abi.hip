@@ -415,6 +415,37 @@ void syn_fwd_ws(C& c, int T, int B, int N, int L, bool hybrid, bool bf16, int ta
     if (hybrid && bf16) c.template take<uint32_t>((size_t)N * N);   // packed W^T | offsets^T
 }
 
+// The blocked hybrid backward (hybblock.hip): N <= 1024 with the offsets' range known, unless a
+// switch asks for another form. `early`: how many steps before the first possible lag 1 the
+// earliest tap of positive weight may start (0 where every lag is >= 1).
+bool hyb_block_on(int N, bool hybrid, int offc) {
+    const char* hs = getenv("DELREC_SYN_HYBSTEP");
+    const char* ls = getenv("DELREC_SYN_LAGSTEP");
+    return hybrid && offc > 0 && N <= 1024 && getenv_flag_off("DELREC_SYN_BWD_HYB_G") &&
+           getenv_flag_off("DELREC_SYN_BWD_HYB") && !(hs && hs[0] == '1') && !(ls && ls[0] == '1');
+}
+
+// the longest early run for a smallest delay (rounded up to the compiled 1, 2, 4, 8; a little
+// slack, so that the device's own fp32 first lag is never below it); 16: longer than compiled
+int hyb_block_early(float d_min, float s, bool lags_ok) {
+    if (lags_ok) return 1;
+    const double lo = std::floor(1.0 + (double)d_min - (double)s - 1e-3) + 1.0;
+    const double run = lo < 1.0 ? 2.0 - lo : 1.0;
+    return run <= 2.0 ? 2 : run <= 4.0 ? 4 : run <= 8.0 ? 8 : 16;
+}
+
+// Where every lag is >= 1 and the runs are compiled (KT 2 or 4), syn_bwd_hyb_g sums each step's
+// G whole, in the step, with one barrier; the blocked scan has a second barrier per step and sums
+// the sources that start below lag 4 step by step, but fetches and decodes a connection once per
+// 4 steps. Measured (scan, T96 B64, sigma 0, 5 offsets; syn_bwd_hyb_g / blocked, us):
+//   fp32 W:  N 96 127 / 142   N 160 225 / 220   N 256 478 / 226   N 512 1662 / 680
+//   bf16 W, delays to 30:  N 160 181 / 198   N 256 258 / 214   N 336 407 / 421   N 512 709 / 626
+//   bf16 W, delays to 14:  N 160 181 / 199   N 256 258 / 264   N 336 407 / 494   N 512 708 / 679
+// (the blocked scan works in quarters of 64 receivers: N just past 256 pays for padding).
+bool hyb_block_pays(int N, int L, bool bf16) {
+    return bf16 ? L >= 28 && ((N >= 208 && N <= 256) || N >= 400) : N >= 176;
+}
+
 template <class C>
 void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf16, int offc, bool lags_ok) {
     // sized for the widest tap run, so the ring may always go to the workspace
@@ -429,6 +460,12 @@ void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf
     c.template take<uint4>(packed);                     // gr_lo
     c.template take<uint4>(packed);                     // shifted spikes
     c.template take<int>((size_t)4 * N + 64);           // lag range per column, meta
+    if (hyb_block_on(N, hybrid, offc)) {
+        const HybBlkShape hb = hyb_block_shape(N, L, bf16, true, 1, 1, 1, (size_t)max_lds_bytes());
+        c.template take<uint4>(hb.wq);                  // packed weights
+        c.template take<uint4>(hb.oq);                  // packed offsets
+        c.template take<int>((size_t)2 * N);            // sources in first-lag order, and its inverse
+    }
     if (syn_hybstep(T, B, N, L, hybrid, offc, taps, lags_ok)) {
         hybstep_ws(c, T, B, N, L, offc, taps, false, bf16);
         return;
@@ -1151,6 +1188,22 @@ int delrec_readout_ce(const delrec_readout_ce_args* a, void* stream) {
     return finish_launch();
 }
 
+// after the reverse scan: the batch sum of db, then the lag correlation folded into dW, dd, ds
+static int syn_bwd_finish(const delrec_syn_bwd_args* a, LagBf16& g, const float* gr, const float* part, int KS,
+                          hipStream_t s) {
+    int st = finish_launch();
+    if (st) return st;
+    launch_reduce_rows(part, a->B, a->N, a->db, nullptr, nullptr, s);
+    if (a->dW || a->dd || a->ds) {
+        launch_lag_bf16(g, a->drop ? gr : a->dx, a->bits, s);
+        LagGemm f{};
+        f.N = a->N; f.KS = KS; f.W = a->W; f.w_bf16 = a->w_bf16; f.s = a->s; f.s_uniform = a->s_uniform;
+        f.pw = g.pw; f.pd = g.pd; f.ps = g.ps; f.perm = lag_bf16_perm(g); f.cls = lag_bf16_cls(g);
+        launch_lag_finish(f, a->dW, a->dd, a->ds, s);
+    }
+    return finish_launch();
+}
+
 int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     if (!a || a->T <= 0 || a->B <= 0 || a->N <= 0 || a->L < 1) return DELREC_ERR_ARG;
     if (!a->gy || !a->u || !a->bits || !a->W || !a->dx || !lif_ok(a->lif)) return DELREC_ERR_ARG;
@@ -1180,15 +1233,33 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     uint4* yb = cv.take<uint4>(packed);
     int* meta = cv.take<int>((size_t)4 * N + 64);
     const int taps = lag_taps(hybrid ? a->s_uniform : (a->s ? a->s_max : std::max(a->s_max, a->s_uniform)));
-    const bool hybstep = syn_hybstep(T, B, N, a->L, hybrid && !a->s, a->off_count, taps,
-                                     a->d_min >= a->s_uniform - 1.0f);
-    const bool lagstep = !hybstep && syn_lagstep(T, B, N, a->L, taps);
+    const bool lags_ok = a->d_min >= a->s_uniform - 1.0f;
+    HybBlk hbp{};
+    HybBlkShape hb{};
+    if (hyb_block_on(N, hybrid, a->off_count)) {
+        hb = hyb_block_shape(N, a->L, a->w_bf16 != 0, true, a->off_count, taps,
+                             hyb_block_early(a->d_min, a->s_uniform, lags_ok), (size_t)max_lds_bytes());
+        const HybBlkShape room = hyb_block_shape(N, a->L, a->w_bf16 != 0, true, 1, 1, 1, (size_t)max_lds_bytes());
+        uint4* wq = cv.take<uint4>(room.wq);
+        uint4* oq = cv.take<uint4>(room.oq);
+        int* ord = cv.take<int>((size_t)2 * N);
+        if (!wq || !oq || !ord) return DELREC_ERR_WORKSPACE;
+        hbp.wq = wq; hbp.oq = oq; hbp.order = ord; hbp.rank = ord + N;
+        if (hb.ok && lags_ok && (KT == 2 || KT == 4) && !hyb_block_pays(N, a->L, a->w_bf16 != 0)) {
+            int gs = 0;
+            const size_t lds_g = syn_bwd_hyb_g_lds(N, a->L, a->off_count, &gs);
+            const size_t lds_t = (size_t)((N + 63) / 64 * 64) * lay.RP * sizeof(float);
+            if (lds_g && std::max(lds_g, lds_t) <= (size_t)max_lds_bytes()) hb.ok = false;
+        }
+    }
+    const bool hybstep = !hb.ok && syn_hybstep(T, B, N, a->L, hybrid && !a->s, a->off_count, taps, lags_ok);
+    const bool lagstep = !hb.ok && !hybstep && syn_lagstep(T, B, N, a->L, taps);
     void* wt = nullptr;
     void* dt = nullptr;
     float* gring = nullptr;
     uint8_t* offq = nullptr;
     int* order = nullptr;
-    if (!lagstep && !hybstep) {
+    if (!lagstep && !hybstep && !hb.ok) {
         wt = cv.take<float>((size_t)N * wlay.NT);
         dt = cv.take<float>((size_t)N * wlay.NT);
         gring = cv.take<float>((size_t)B * N * wlay.RP);
@@ -1206,9 +1277,9 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     // laid out in that order, so a lane's runs stay adjacent to its neighbours'.
     const size_t hrows = (size_t)((N + 63) / 64 * 64);
     const size_t lds_h = hrows * lay.RP * sizeof(float);
-    const bool hyb_fast = hybrid && !lagstep && !hybstep && N <= 512 && (lay.KT == 2 || lay.KT == 4) &&
+    const bool hyb_fast = hybrid && !lagstep && !hybstep && !hb.ok && N <= 512 && (lay.KT == 2 || lay.KT == 4) &&
                           lds_h <= (size_t)max_lds_bytes() && getenv_flag_off("DELREC_SYN_BWD_HYB");
-    if (!lagstep && !hybstep) {
+    if (!lagstep && !hybstep && !hb.ok) {
         if (hyb_fast) launch_sort_by_first_lag(a->base, a->s_uniform, N, order, s);
         const int* ord = hyb_fast ? order : nullptr;
         if (a->w_bf16) block_transpose<uint16_t>(a->W, wt, N, s, ord); else block_transpose<float>(a->W, wt, N, s, ord);
@@ -1228,7 +1299,7 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     g.pd = lagp + (size_t)q.KS * NN;
     g.ps = a->ds ? lagp + (size_t)2 * q.KS * NN : nullptr;
     launch_lag_cols(g, s);
-    if (hybrid && !lagstep && !hybstep) launch_pack_offq(static_cast<const int8_t*>(dt), (size_t)N * lay.NT, meta, offq, s);
+    if (hybrid && !lagstep && !hybstep && !hb.ok) launch_pack_offq(static_cast<const int8_t*>(dt), (size_t)N * lay.NT, meta, offq, s);
 
     if (hybstep) {
         // reverse-time scan in blocks of P steps, the sources split by first lag: far ones
@@ -1486,6 +1557,20 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
         return finish_launch();
     }
 
+    if (hb.ok) {
+        hbp.T = T; hbp.B = B; hbp.N = N; hbp.NCl = hb.NCl; hbp.Ns = hb.Ns; hbp.RG = hb.RG;
+        hbp.KF = taps; hbp.D = hb.Dmax; hbp.room = hb.room; hbp.nwg = hb.nwg; hbp.gy = a->gy; hbp.u = a->u; hbp.base = a->base; hbp.meta = meta;
+        hbp.s_uniform = a->s_uniform; hbp.drop = a->drop; hbp.lif = make_lif(a->lif);
+        hbp.dx = a->dx; hbp.gr = a->drop ? gr : nullptr; hbp.part = part;
+        launch_hyb_block_pack(hbp, const_cast<uint4*>(hbp.wq), const_cast<uint4*>(hbp.oq),
+                              const_cast<int*>(hbp.order), const_cast<int*>(hbp.rank), a->W, a->offsets, a->w_bf16 != 0, s);
+        const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
+        const bool ok = launch_hyb_block_bwd(hbp, hb, a->w_bf16 != 0, s);
+        scan_end(timed && ok, s);
+        if (!ok) return DELREC_ERR_UNSUPPORTED;
+        return syn_bwd_finish(a, g, gr, part, q.KS, s);
+    }
+
     SynBwd p{};
     p.T = T; p.B = B; p.N = N; p.L = a->L;
     p.R = lay.R; p.RS = lay.RS; p.RP = lay.RP; p.KT = lay.KT; p.NT = lay.NT;
@@ -1514,17 +1599,7 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     const bool ok = hyb_g || (hyb_fast ? launch_syn_bwd_hyb(p, lay.block, lds_hx, s) : launch_syn_bwd(p, lay.block, lay.lds, s));
     scan_end(timed && ok, s);
     if (!ok) return DELREC_ERR_UNSUPPORTED;
-    int st = finish_launch();
-    if (st) return st;
-    launch_reduce_rows(part, B, N, a->db, nullptr, nullptr, s);
-    if (a->dW || a->dd || a->ds) {
-        launch_lag_bf16(g, a->drop ? gr : a->dx, a->bits, s);
-        LagGemm f{};
-        f.N = N; f.KS = q.KS; f.W = a->W; f.w_bf16 = a->w_bf16; f.s = a->s; f.s_uniform = a->s_uniform;
-        f.pw = g.pw; f.pd = g.pd; f.ps = g.ps; f.perm = lag_bf16_perm(g); f.cls = lag_bf16_cls(g);
-        launch_lag_finish(f, a->dW, a->dd, a->ds, s);
-    }
-    return finish_launch();
+    return syn_bwd_finish(a, g, gr, part, q.KS, s);
 }
 
 int delrec_lif_fwd(const delrec_lif_fwd_args* a, void* stream) {

@@ -107,6 +107,36 @@ struct SynBwd {
     const uint8_t* offq;        // blocked (offset - smallest offset) * 4 as bytes (hybrid), or NULL
 };
 
+// The blocked reverse scan of hybrid and wide axonal layers (hybblock.hip).
+struct HybBlkShape {
+    bool ok;
+    int NPL, nwg, NCl, Ns, block;   // neurons per lane, waves that sum, chunks of 16 receivers per lane, source slots, threads
+    int R, NT, RG, Dmax, room;  // gr ring slots, slots of a near sum, G history slots, offsets the ring holds, near partials' floats
+    size_t lds, wq, oq;         // LDS bytes, uint4 of the packed weights and offsets
+};
+struct HybBlk {
+    int T, B, N, NCl, Ns, RG, KF, D, room, nwg;
+    const float* gy;
+    const float* u;
+    const uint4* wq;
+    const uint4* oq;            // packed offsets, or NULL (axonal)
+    const float* base;          // hybrid base, or the axonal delays
+    const int* order;           // sources in first-lag order
+    const int* rank;            // and its inverse
+    const int* meta;            // meta[1], meta[2] = smallest and largest offset, or NULL
+    float s_uniform;
+    const float* drop;
+    Lif lif;
+    float* dx;
+    float* gr;                  // (T,B,N), or NULL where it equals dx
+    float* part;                // [B][N] db partials
+    float* gz;                  // (T,B,N) G, or NULL
+};
+HybBlkShape hyb_block_shape(int N, int L, bool bf16, bool offsets, int D, int KF, int NT, size_t max_lds);
+void launch_hyb_block_pack(const HybBlk& p, uint4* wq, uint4* oq, int* order, int* rank, const void* W,
+                           const int8_t* off, bool bf16, hipStream_t s);
+bool launch_hyb_block_bwd(const HybBlk& p, const HybBlkShape& q, bool bf16, hipStream_t s);
+
 // the split partials of the lag GEMM and what dd / ds are formed from
 struct LagGemm {
     int N, KS;

@@ -1,0 +1,80 @@
+"""The blocked reverse scan of hybrid delays (``hybblock.hip``) against the float64 oracle, at
+the sizes where its groups, chunks, blocks and ring runs have edges: one group and a partial
+one, a quarter of the receivers more and less than whole chunks of 16, one, two and four
+neurons per lane, far groups dealt out over more than one round; early runs of 2, 4 and 8
+slots (half-widths over 1 near the delay 0, negative bases), more than 9 offsets (the wider
+ring), every source near, steps that are no multiple of a block, tap counts past four; and,
+with a dropout mask and a bias, against the per-tap gather. Tolerances: ``tests/helpers.py``."""
+
+import pytest
+import torch
+
+from test_gpu_synaptic import test_hybrid_fwd_bwd_matches_oracle as check_case
+from test_gpu_synaptic import hybrid_layer
+from helpers import gen
+
+CASES = [
+    # T, B, N, base range, max offset, bf16 weights, sigma
+    (21, 2, 16, (0.0, 9.0), 4, False, 1.0),
+    (22, 3, 17, (0.0, 14.0), 3, True, 1.0),
+    (23, 2, 63, (0.0, 24.0), 8, True, 3.0),
+    (24, 2, 65, (-3.0, 12.0), 2, False, 3.0),       # early runs of 8
+    (25, 2, 130, (0.0, 30.0), 11, False, 1.0),      # 12 offsets: the ring of 32 slots
+    (26, 2, 192, (0.0, 2.5), 4, False, 0.0),        # every source near
+    (27, 2, 193, (0.0, 26.0), 4, True, 0.4),
+    (28, 2, 256, (0.0, 33.0), 8, False, 1.0),
+    (29, 2, 257, (0.0, 20.0), 4, False, 0.0),
+    (30, 2, 385, (0.0, 28.0), 5, True, 2.5),
+    (31, 1, 513, (0.0, 18.0), 3, False, 1.0),
+    (22, 1, 600, (0.0, 12.0), 2, True, 0.0),
+    (20, 2, 48, (0.0, 10.0), 3, False, 4.0),        # ten taps
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', CASES, ids=[f'T{c[0]}N{c[2]}K{c[4]}{"bf16" if c[5] else ""}s{c[6]}' for c in CASES])
+def test_blocked_backward_matches_oracle(dev, case):
+    check_case(dev, case)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('N', [96, 260])
+def test_blocked_backward_repeats_bit_for_bit(dev, N):
+    """Two passes on the same inputs: partial sums meet in a fixed order."""
+    g = gen(3)
+    T, B = 33, 5
+    layer = hybrid_layer(N, torch.randn(N, N, generator=g) / N ** 0.5, torch.rand(N, generator=g) * 20,
+                         torch.randint(5, (N, N), generator=g).float(), dev, bf16=False, sigma_init=1.0)
+    x, gy = torch.randn(T, B, N, generator=g).to(dev), torch.randn(T, B, N, generator=g).to(dev)
+    out = []
+    for _ in range(2):
+        layer.zero_grad(set_to_none=True)
+        xi = x.clone().requires_grad_(True)
+        layer(xi).backward(gy)
+        out.append([xi.grad] + [p.grad for p in layer.parameters()])
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.gpu
+def test_blocked_backward_with_dropout_and_bias(dev, monkeypatch):
+    """The same pass through ``syn_bwd_kernel``: the sums differ by their order (up to N terms of
+    2^-24 each; 1e-5 of the largest value)."""
+    from delrec.kernels import HybridSynDelay
+    g = gen(4)
+    T, B, N = 27, 3, 200
+    layer = hybrid_layer(N, torch.randn(N, N, generator=g) / N ** 0.5, torch.rand(N, generator=g) * 15,
+                         torch.randint(6, (N, N), generator=g).float(), dev, bf16=False, sigma_init=1.0)
+    drop = (torch.rand(B, N, generator=g) > 0.3).float().to(dev) / 0.7
+    x, gy = torch.randn(T, B, N, generator=g).to(dev), torch.randn(T, B, N, generator=g).to(dev)
+    bias = (torch.randn(N, generator=g) * 0.1).to(dev)
+    out = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setenv('DELREC_SYN_BWD_HYB', '0')
+        layer.zero_grad(set_to_none=True)
+        xi, bi = x.clone().requires_grad_(True), bias.clone().requires_grad_(True)
+        HybridSynDelay.apply(xi, layer.recurrent_weights, layer.recurrent_delays, bi, drop, layer).backward(gy)
+        out.append([xi.grad, bi.grad] + [p.grad for p in layer.parameters()])
+    for a, b in zip(*out):
+        torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
