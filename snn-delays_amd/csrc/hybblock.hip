@@ -19,12 +19,14 @@
 //     yet formed hold 0, so these are the same run of slots, started earlier.
 //
 // Bound: the LDS reads of gr (4 bytes per connection and step at 128 B/clk: 2,048 clk a step at
-// N = 256, 8,192 at N = 512) beside the issue of the multiply-adds, then the two exchanges of a
-// step. Measured (scan): T250 B128 N256 sigma 1, 5 offsets, fp32 W 0.65 ms, 2.6 us a step (23.5 ms
-// with the per-tap gather of syn_bwd_kernel); T256 B256 N512 sigma 0, 9 offsets, bf16 W 1.83 ms
-// (2.22 ms with syn_bwd_hyb_g). A group's whole block taken in one step by its own wave alone:
-// 5.2 ms there (one wave per SIMD at a time hides nothing); neurons on the summing waves
-// instead of waves of their own: 1.1 and 2.0 ms (their registers together spill).
+// N = 256, 8,192 at N = 512; without offsets one read serves 16 receivers' multiply-adds, whose
+// issue, 4,096 clk at N = 512, is the bound then) and the two exchanges of a step.
+// Measured (scan): T250 B128 N256 sigma 1, 5 offsets, fp32 W 0.65 ms, 2.6 us a step (23.5 ms with
+// the per-tap gather of syn_bwd_kernel); T256 B256 N512 sigma 0, 9 offsets, bf16 W 1.8 ms (2.22 ms
+// with syn_bwd_hyb_g); axonal T250 B256 N512 sigma 1 fp32 W 1.4 ms (8.70 ms with the dense
+// product streamed per step, axonal_bwd_kernel). A group's whole block taken in one step by its
+// own wave alone: 5.2 ms at N = 512 (one wave per SIMD at a time hides nothing); neurons on the
+// summing waves instead of waves of their own: 2.0 ms (their registers together spill).
 #include <algorithm>
 
 #include "common.h"
@@ -43,6 +45,43 @@ __device__ __forceinline__ int first_lag(float c, float s) {
     if (fabsf((float)lo - c) > s) lo += 1;
     if (s - fabsf((float)lo - c) <= 0.0f) lo += 1;
     return lo;
+}
+
+// acc[n] += sum over q < 4 of w[q] * (g[n] of lane E + q of the lane's row of 16): the broadcast is
+// an operand modifier of the multiply-add (the compiler makes it a move of its own). The s_nop
+// covers the two wait states a row-modified operand needs after a vector write.
+template <int E>
+__device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[1], float (&acc)[1]) {
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %1, %2 row_newbcast:%6 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %3 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %4 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
+        : "+v"(acc[0])
+        : "v"(g[0]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(E), "n"(E + 1), "n"(E + 2), "n"(E + 3));
+}
+
+#define DELREC_FMAC2(W, E)                                                      \
+    "v_fmac_f32_dpp %0, %2, " W " row_newbcast:" E " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %1, %3, " W " row_newbcast:" E " row_mask:0xf bank_mask:0xf\n\t"
+template <int E>
+__device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[2], float (&acc)[2]) {
+    asm("s_nop 1\n\t" DELREC_FMAC2("%4", "%8") DELREC_FMAC2("%5", "%9") DELREC_FMAC2("%6", "%10") DELREC_FMAC2("%7", "%11")
+        : "+v"(acc[0]), "+v"(acc[1])
+        : "v"(g[0]), "v"(g[1]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(E), "n"(E + 1), "n"(E + 2), "n"(E + 3));
+}
+
+#define DELREC_FMAC4(W, E)                                                      \
+    "v_fmac_f32_dpp %0, %4, " W " row_newbcast:" E " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %1, %5, " W " row_newbcast:" E " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %2, %6, " W " row_newbcast:" E " row_mask:0xf bank_mask:0xf\n\t" \
+    "v_fmac_f32_dpp %3, %7, " W " row_newbcast:" E " row_mask:0xf bank_mask:0xf\n\t"
+template <int E>
+__device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[4], float (&acc)[4]) {
+    asm("s_nop 1\n\t" DELREC_FMAC4("%8", "%12") DELREC_FMAC4("%9", "%13") DELREC_FMAC4("%10", "%14") DELREC_FMAC4("%11", "%15")
+        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
+        : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(E), "n"(E + 1),
+          "n"(E + 2), "n"(E + 3));
 }
 
 }  // namespace
@@ -118,7 +157,7 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
     constexpr int WV = WBF ? 2 : 4;                        // uint4 of W per chunk
     constexpr int CPW = 16 / WV;                           // receivers per uint4 of W
     constexpr uint32_t MB = R * 4 - 1;                     // byte offset within the R slots
-    constexpr int PAD = R == 16 ? 16 : 32;                 // words between the quarters
+    constexpr int PAD = R <= 16 ? 16 : 32;                 // words between the quarters
     constexpr int PF = 2;                                  // steps of gy / u loaded ahead
     static_assert(NT <= PITCH - R + 1 && PITCH - R >= 3, "runs of slots past the repeated ones");
     const int N = p.N, T = p.T, B = p.B, Ns = p.Ns, NCl = p.NCl, RG = p.RG;
@@ -135,10 +174,7 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
     };
     // groups in first-lag order: near ones first
     const int glo = tid < ngroups ? lag_of(p.order[tid * 16]) : 0x7fffffff;
-    int nn = __syncthreads_count(glo < 4);
-    // (a round of far groups that would keep one or two waves only is summed as near ones)
-    const int over = (ngroups - nn) % nw;
-    if (ngroups - nn > nw && over <= 2) nn += over;
+    const int nn = __syncthreads_count(glo < 4);
     // a caller's claims that the device data contradict (offsets past the stated range, a
     // source that starts earlier than the smallest delay it gave) make every output NaN
     const bool wrong = OFF && (D > p.D || __syncthreads_or(glo < 2 - NT) != 0);
@@ -186,7 +222,8 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
     };
     // the operands of the next chunk to sum
     struct Chunk { uint4 w[WV], o; };
-    Chunk nearc, farc;
+    constexpr bool DEEP = GPW > 1 && !OFF;                 // registers for a second chunk of each
+    Chunk nearc, nears, farc, fars;
     auto fetch_w = [&](Chunk& ch, int h, int gb, int c) { ch.w[h] = load4(rw, wl, ((c * WV + h) * Ns + gb) * 16); };
     auto fetch_o = [&](Chunk& ch, int gb, int c) {
         if constexpr (OFF) ch.o = load4(ro, ol, (c * Ns + gb) * 16);
@@ -203,6 +240,35 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
         constexpr int NP = sizeof(acc) / sizeof(float);
         constexpr int GR = NP >= 4 ? 2 : 4;                // receivers read together
         const uint32_t cb = rowb + (uint32_t)c * (16 * PITCH * 4);
+        if constexpr (!OFF) {
+            // every source reads the same slots: lane `src` reads receiver src's, and each
+            // multiply-add takes its receiver's value from that lane of the row
+            float g[NP];
+            const auto* x = (const __attribute__((address_space(3))) float*)(uintptr_t)(cb + st + (uint32_t)src * (PITCH * 4));
+#pragma unroll
+            for (int n = 0; n < NP; ++n) g[n] = x[n];
+            auto four = [&](auto e0) {                     // receivers E .. E + 3
+                constexpr int E = decltype(e0)::value;
+                float wf[4];
+                if constexpr (WBF) {
+                    const uint4& v = ch.w[E >> 3];
+                    const uint32_t a = E & 4 ? v.z : v.x, b2 = E & 4 ? v.w : v.y;
+                    wf[0] = __uint_as_float(a << 16); wf[1] = __uint_as_float(a & 0xFFFF0000u);
+                    wf[2] = __uint_as_float(b2 << 16); wf[3] = __uint_as_float(b2 & 0xFFFF0000u);
+                } else {
+                    const uint4& v = ch.w[E >> 2];
+                    wf[0] = __uint_as_float(v.x); wf[1] = __uint_as_float(v.y);
+                    wf[2] = __uint_as_float(v.z); wf[3] = __uint_as_float(v.w);
+                }
+                add_rows<E>(wf, g, acc);
+                if ((E + 4) % CPW == 0 && refill) fetch_w(ch, E / CPW, ngb, nc);
+            };
+            four(std::integral_constant<int, 0>{});
+            four(std::integral_constant<int, 4>{});
+            four(std::integral_constant<int, 8>{});
+            four(std::integral_constant<int, 12>{});
+            return;
+        }
         // four slots of connections at a time: no byte carries over (both summands < 128)
         uint4 oc = make_uint4(st, st, st, st);
         if constexpr (OFF) {
@@ -313,45 +379,56 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
             const bool live = t >= 0;
             if (r == 0) load_steps(t - PF, gn, un);
             barrier_lds();
+            // near sources' sums, and below lag 1 the taps on the truncated ones (all the lane's
+            // neurons at each stage: one LDS round trip for all of them)
+            float v[NPL][NT][4], gfs[NPL], gnear[NPL];
 #pragma unroll
-            for (int i = 0; i < NPL; ++i) {
-                const int j = max(jn[i], 0);
-                // near sources' sums, and below lag 1 the taps on the truncated ones
-                float v[NT][4];
+            for (int i = 0; i < NPL; ++i)
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) v[n][q] = mine[i][((q < slices ? q : 0) * NT + n) * 16];
-                float gf = 0.0f, a[NT];
+                    for (int q = 0; q < 4; ++q) v[i][n][q] = mine[i][((q < slices ? q : 0) * NT + n) * 16];
+#pragma unroll
+            for (int i = 0; i < NPL; ++i) {
+                gfs[i] = 0.0f;
 #pragma unroll
                 for (int n = 0; n < NT; ++n) {
-                    a[n] = v[n][0];
+                    float a = v[i][n][0];
 #pragma unroll
-                    for (int q = 1; q < 4; ++q) a[n] += q < slices ? v[n][q] : 0.0f;
+                    for (int q = 1; q < 4; ++q) a += q < slices ? v[i][n][q] : 0.0f;
                     if (n < NT - 1)
-                        gf = fmaf(fmaxf(sv - fabsf((float)(n + 2 - NT - omin) - cn[i]), 0.0f), near_j[i] ? a[n] : 0.0f, gf);
+                        gfs[i] = fmaf(fmaxf(sv - fabsf((float)(n + 2 - NT - omin) - cn[i]), 0.0f), near_j[i] ? a : 0.0f, gfs[i]);
+                    gnear[i] = a;
                 }
-                if (near_j[i]) {
-                    ghist[__umul24(g1, Ns) + j] = a[NT - 1];
-                    keep_gz(t + 1, j, a[NT - 1]);
-                }
-                // (four taps at a time: the weights are formed here and not held in registers; a tap
-                // past the triangle weighs 0)
+            }
+#pragma unroll
+            for (int i = 0; i < NPL; ++i)
+                if (near_j[i]) ghist[__umul24(g1, Ns) + jn[i]] = gnear[i];
+            // (four taps at a time: the weights are formed here and not held in registers; a tap past
+            // the triangle weighs 0)
 #pragma unroll 1
-                for (int f0 = 0; f0 < p.KF; f0 += 4) {
-                    float gv[4];
+            for (int f0 = 0; f0 < p.KF; f0 += 4) {
+                float gv[NPL][4];
+#pragma unroll
+                for (int i = 0; i < NPL; ++i)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        int sl = g1 + max(lon[i] + f0 + q, 1) - 1;
+                        int sl = g1 + min(max(lon[i] + f0 + q, 1), RG - 1) - 1;
                         sl = sl >= RG ? sl - RG : sl;
-                        gv[q] = ghist[__umul24(sl, Ns) + j];
+                        gv[i][q] = ghist[__umul24(sl, Ns) + max(jn[i], 0)];
                     }
+#pragma unroll
+                for (int i = 0; i < NPL; ++i)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         const float h = fmaxf(sv - fabsf(x0[i] + (float)(f0 + q)), 0.0f);
-                        gf = fmaf(lon[i] + f0 + q >= 1 ? h : 0.0f, gv[q], gf);
+                        gfs[i] = fmaf(lon[i] + f0 + q >= 1 ? h : 0.0f, gv[i][q], gfs[i]);
                     }
-                }
+            }
+#pragma unroll
+            for (int i = 0; i < NPL; ++i) {
+                if (near_j[i]) keep_gz(t + 1, jn[i], gnear[i]);
+                float gf = gfs[i];
                 gf *= is2;
                 const float u = r == 0 ? uq[i][0] : uq[i][1], gyv = r == 0 ? gq[i][0] : gq[i][1];
                 const float y = lif_fire(k, u);
@@ -398,11 +475,17 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
     for (int q = 0; q < GPW; ++q)
 #pragma unroll
         for (int n = 0; n < 4; ++n) acc[q][n] = 0.0f;
-    // the wave's first near unit; whether it is all its near work, one chunk: it stays loaded
+    // the wave's first near unit; whether it is all its near work, one chunk or two: it stays loaded
     const int u_gb = wave / slices * 16, u_c = min(wave % slices * per_slice, NCl - 1);
-    const bool one = per_slice == 1 && wave + nw >= units;
+    const bool one = per_slice <= (DEEP ? 2 : 1) && wave + nw >= units;
+    const bool both = per_slice == 2 && u_c + 1 < NCl;
     if (wave < units) fetch(nearc, u_gb, u_c);
-    if (nfar > 0) fetch(farc, far_group(0) * 16, min(far_first(0, T - 1), NCl - 1));
+    if (DEEP && wave < units && both) fetch(nears, u_gb, u_c + 1);
+    if (nfar > 0) {
+        const int c = min(far_first(0, T - 1), NCl - 1);
+        fetch(farc, far_group(0) * 16, c);
+        if constexpr (DEEP) fetch(fars, far_group(0) * 16, min(c + 1, NCl - 1));
+    }
     __syncthreads();
     for (int t = T - 1; t >= tend; --t) {
         for (int u = wave; u < units; u += nw) {
@@ -411,7 +494,12 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
             for (int n = 0; n < NT; ++n) cur[n] = 0.0f;
             const uint32_t st = ((uint32_t)(t + 2 - NT) * 4u) & MB;
             if (one) {
-                if (wave % slices < NCl) sum_chunk(nearc, u_c, st, false, 0, 0, cur);
+                if (wave % slices * per_slice < NCl) {
+                    sum_chunk(nearc, u_c, st, false, 0, 0, cur);
+                    if constexpr (DEEP) {
+                        if (both) sum_chunk(nears, u_c + 1, st, false, 0, 0, cur);
+                    }
+                }
             } else {
                 const int g = u / slices, sl = u - g * slices;
                 const int c0 = min(sl * per_slice, NCl), c1 = min(c0 + per_slice, NCl);
@@ -451,17 +539,30 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
                         for (int n = 0; n < 4; ++n) cur[n] = acc[x][n];
                     }
             }
-#pragma unroll 1
-            for (int c = c0; c < c1; ++c) {
-                const bool last = c + 1 == c1;
-                const int ngb = last ? gx : far_group(q) * 16, nc = last ? cx : min(c + 1, NCl - 1);
+            auto sum_far = [&](Chunk& ch, int c, int ngb, int nc) {
                 if (c >= NCl) {                            // (the last step of a block may have fewer)
-                    if (last) fetch(farc, ngb, nc);
+                    fetch(ch, ngb, min(nc, NCl - 1));
                 } else if (p4) {
-                    sum_chunk(farc, c, st, true, ngb, nc, cur);
+                    sum_chunk(ch, c, st, true, ngb, min(nc, NCl - 1), cur);
                 } else {
                     float (&c2)[2] = reinterpret_cast<float (&)[2]>(cur);
-                    sum_chunk(farc, c, st, true, ngb, nc, c2);
+                    sum_chunk(ch, c, st, true, ngb, min(nc, NCl - 1), c2);
+                }
+            };
+            if constexpr (DEEP) {                          // chunks in pairs, the next pair on its way
+#pragma unroll 1
+                for (int c = c0; c < c1; c += 2) {
+                    const bool last = c + 2 >= c1;
+                    const int ngb = last ? gx : far_group(q) * 16, nc = last ? cx : c + 2;
+                    sum_far(farc, c, ngb, nc);
+                    if (c + 1 < c1) sum_far(fars, c + 1, ngb, nc + 1);
+                    else if (last) fetch(fars, ngb, min(nc + 1, NCl - 1));
+                }
+            } else {
+#pragma unroll 1
+                for (int c = c0; c < c1; ++c) {
+                    const bool last = c + 1 == c1;
+                    sum_far(farc, c, last ? gx : far_group(q) * 16, last ? cx : c + 1);
                 }
             }
             if (sub != P - 1) {
@@ -508,7 +609,7 @@ bool launch_one(const HybBlk& p, const HybBlkShape& q, hipStream_t s) {
 template <int GPW, int NPL, bool WBF>
 bool launch_ring(const HybBlk& p, const HybBlkShape& q, hipStream_t s) {
     if (!p.oq) {
-        if constexpr (GPW > 1) return launch_one<GPW, NPL, WBF, false, 16, 20, 1>(p, q, s);
+        if constexpr (GPW > 1) return launch_one<GPW, NPL, WBF, false, 8, 12, 1>(p, q, s);
         return false;
     }
     if (q.R == 32) return launch_one<GPW, NPL, WBF, true, 32, 40, 8>(p, q, s);
@@ -524,9 +625,9 @@ HybBlkShape hyb_block_shape(int N, int L, bool bf16, bool offsets, int D, int KF
     if (N < 1 || N > 1024 || D < 1 || KF < 1 || KF > kTapsMax || NT > 8) return q;
     // steps whose slots must differ: t - NT + 1 (early run) .. t + 7 (spread block of 4 steps) and
     // the D - 1 offsets
-    q.R = 6 + NT + D <= 16 && NT <= 4 ? 16 : 6 + 8 + D <= 32 ? 32 : 0;
-    if (!q.R || (!offsets && q.R != 16)) return q;
-    q.NT = q.R == 16 ? NT : 8;
+    q.R = !offsets ? 8 : 6 + NT + D <= 16 && NT <= 4 ? 16 : 6 + 8 + D <= 32 ? 32 : 0;
+    if (!q.R) return q;
+    q.NT = q.R <= 16 ? NT : 8;
     q.Dmax = q.R - 6 - q.NT;
     const int groups = (N + 15) / 16;
     q.NPL = N <= 192 ? 1 : N <= 384 ? 2 : 4;
@@ -535,14 +636,14 @@ HybBlkShape hyb_block_shape(int N, int L, bool bf16, bool offsets, int D, int KF
     q.nwg = std::min(16 - neuron_waves, std::max(groups * std::min(q.NCl, 4), 4));   // far groups per wave: at most 1, 2, 2, 3, 6
     q.block = (q.nwg + neuron_waves) * 64;
     q.Ns = groups * 16;
-    q.RG = std::max(L + 4, 9);
-    const int pitch = q.R == 16 ? 20 : 40, pad = q.R == 16 ? 16 : 32;
+    q.RG = std::max(L, 8) + 1;                             // steps t + 1 .. t + L - 1, blocks to t + 7
+    const int pitch = q.R == 8 ? 12 : q.R == 16 ? 20 : 40, pad = q.R <= 16 ? 16 : 32;
     const size_t words = (size_t)4 * (q.NCl * 16 * pitch + pad) + 64 + (size_t)q.RG * q.Ns;
     // near partials: one slice of every group at least, up to 16 KB
     const size_t least = (size_t)q.Ns * q.NT;
     q.wq = (size_t)4 * q.NCl * (bf16 ? 2 : 4) * q.Ns;
     q.oq = offsets ? (size_t)4 * q.NCl * q.Ns : 0;
-    const size_t avail = (max_lds - 1024) / sizeof(float);   // (block reductions hold some statically)
+    const size_t avail = max_lds / sizeof(float);
     if (words + least > avail || (!offsets && N <= 256)) return q;
     q.room = (int)std::min(avail - words, std::max(least, (size_t)4096));
     q.lds = (words + q.room) * sizeof(float);

@@ -107,6 +107,10 @@ struct SynBwd {
     const uint8_t* offq;        // blocked (offset - smallest offset) * 4 as bytes (hybrid), or NULL
 };
 
+// The axonal forward as a scatter of arriving spikes (axwide.hip): soft taps of one half-width,
+// kf = 2, 4 or 8 >= ceil(2 s) taps, hw = 1, 2 or 4 history words of 64 lags, N <= 1024.
+bool launch_axonal_fwd_arrive(const AxFwd& p, int kf, int hw, hipStream_t stream);
+
 // The blocked reverse scan of hybrid and wide axonal layers (hybblock.hip).
 struct HybBlkShape {
     bool ok;
