@@ -461,6 +461,13 @@ bool hyb_block_pays(int N, int L, bool bf16) {
     return bf16 ? L >= 28 && ((N >= 208 && N <= 256) || N >= 400) : N >= 176;
 }
 
+// The synaptic backward on interpolation tables (synlin.hip): N <= 1024, not under the switches
+// that force the lag-stacked scan or the general one (DELREC_SYN_LIN=0)
+bool syn_lin_on(int N, bool hybrid) {
+    const char* ls = getenv("DELREC_SYN_LAGSTEP");
+    return !hybrid && N <= 1024 && !(ls && ls[0] == '1') && getenv_flag_off("DELREC_SYN_LIN");
+}
+
 template <class C>
 void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf16, int offc, bool lags_ok) {
     // sized for the widest tap run, so the ring may always go to the workspace
@@ -480,6 +487,10 @@ void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf
         c.template take<uint4>(hb.wq);                  // packed weights
         c.template take<uint4>(hb.oq);                  // packed offsets
         c.template take<int>((size_t)2 * N);            // sources in first-lag order, and its inverse
+    }
+    if (syn_lin_on(N, hybrid)) {
+        const SynLinShape sl = syn_lin_shape(N, 2, 1.0f, (size_t)max_lds_bytes());
+        c.template take<uint4>(2 * sl.pack);            // packed weights and delays
     }
     if (syn_hybstep(T, B, N, L, hybrid, offc, taps, lags_ok)) {
         hybstep_ws(c, T, B, N, L, offc, taps, false, bf16);
@@ -1293,14 +1304,25 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
             if (lds_g && std::max(lds_g, lds_t) <= (size_t)max_lds_bytes()) hb.ok = false;
         }
     }
+    // per-connection delays of one half-width whose tables fit LDS: linear interpolation. The
+    // entry's own ring (one value per step) must fit too, so that the lag-stacked scan keeps its
+    // sizes.
+    SynLinShape sl{};
+    uint4* slp = nullptr;
+    if (syn_lin_on(N, hybrid)) {
+        const SynLinShape room = syn_lin_shape(N, 2, 1.0f, (size_t)max_lds_bytes());
+        slp = cv.take<uint4>(2 * room.pack);
+        if (!slp) return DELREC_ERR_WORKSPACE;
+        if (!a->s && lay.lds_ring) sl = syn_lin_shape(N, a->L, a->s_uniform, (size_t)max_lds_bytes());
+    }
     const bool hybstep = !hb.ok && syn_hybstep(T, B, N, a->L, hybrid && !a->s, a->off_count, taps, lags_ok);
-    const bool lagstep = !hb.ok && !hybstep && syn_lagstep(T, B, N, a->L, taps);
+    const bool lagstep = !hb.ok && !sl.ok && !hybstep && syn_lagstep(T, B, N, a->L, taps);
     void* wt = nullptr;
     void* dt = nullptr;
     float* gring = nullptr;
     uint8_t* offq = nullptr;
     int* order = nullptr;
-    if (!lagstep && !hybstep && !hb.ok) {
+    if (!lagstep && !hybstep && !hb.ok && !sl.ok) {
         wt = cv.take<float>((size_t)N * wlay.NT);
         dt = cv.take<float>((size_t)N * wlay.NT);
         gring = cv.take<float>((size_t)B * N * wlay.RP);
@@ -1320,7 +1342,7 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     const size_t lds_h = hrows * lay.RP * sizeof(float);
     const bool hyb_fast = hybrid && !lagstep && !hybstep && !hb.ok && N <= 512 && (lay.KT == 2 || lay.KT == 4) &&
                           lds_h <= (size_t)max_lds_bytes() && getenv_flag_off("DELREC_SYN_BWD_HYB");
-    if (!lagstep && !hybstep && !hb.ok) {
+    if (!lagstep && !hybstep && !hb.ok && !sl.ok) {
         if (hyb_fast) launch_sort_by_first_lag(a->base, a->s_uniform, N, order, s);
         const int* ord = hyb_fast ? order : nullptr;
         if (a->w_bf16) block_transpose<uint16_t>(a->W, wt, N, s, ord); else block_transpose<float>(a->W, wt, N, s, ord);
@@ -1607,6 +1629,19 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
                               const_cast<int*>(hbp.order), const_cast<int*>(hbp.rank), a->W, a->offsets, a->w_bf16 != 0, s);
         const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
         const bool ok = launch_hyb_block_bwd(hbp, hb, a->w_bf16 != 0, s);
+        scan_end(timed && ok, s);
+        if (!ok) return DELREC_ERR_UNSUPPORTED;
+        return syn_bwd_finish(a, g, gr, part, q.KS, s);
+    }
+
+    if (sl.ok) {
+        SynLin p{};
+        p.T = T; p.B = B; p.N = N; p.L = a->L; p.NC = sl.NC; p.Ns = sl.Ns; p.slices = sl.slices; p.per = sl.per;
+        p.m = sl.m; p.R = sl.R; p.w_bf16 = a->w_bf16; p.gy = a->gy; p.u = a->u; p.wq = slp; p.fq = slp + sl.pack;
+        p.s_uniform = a->s_uniform; p.drop = a->drop; p.lif = make_lif(a->lif);
+        p.dx = a->dx; p.gr = a->drop ? gr : nullptr; p.part = part;
+        const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
+        const bool ok = launch_syn_lin_bwd(p, sl, slp, slp + sl.pack, a->W, a->d, s);
         scan_end(timed && ok, s);
         if (!ok) return DELREC_ERR_UNSUPPORTED;
         return syn_bwd_finish(a, g, gr, part, q.KS, s);

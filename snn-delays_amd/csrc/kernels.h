@@ -107,6 +107,30 @@ struct SynBwd {
     const uint8_t* offq;        // blocked (offset - smallest offset) * 4 as bytes (hybrid), or NULL
 };
 
+// The synaptic reverse scan on interpolation tables (synlin.hip): one half-width, windows of up to
+// about 60 lags whose tables fit LDS.
+struct SynLinShape {
+    bool ok, frac;
+    int m, R, NC, Ns, slices, per, block;   // floor(s), slots, chunks of 16 receivers, source slots, receiver slices
+    size_t lds, pack;                        // LDS bytes, uint4 of each packed operand
+};
+struct SynLin {
+    int T, B, N, L, NC, Ns, slices, per, m, R, w_bf16;
+    const float* gy;
+    const float* u;
+    const uint4* wq;
+    const uint4* fq;
+    float s_uniform;
+    const float* drop;
+    Lif lif;
+    float* dx;
+    float* gr;                  // (T,B,N), or NULL where it equals dx
+    float* part;                // [B][N] db partials
+};
+SynLinShape syn_lin_shape(int N, int L, float s, size_t max_lds);
+bool launch_syn_lin_bwd(const SynLin& p, const SynLinShape& q, uint4* wq, uint4* fq, const void* W, const float* d,
+                        hipStream_t s);
+
 // The axonal forward as a scatter of arriving spikes (axwide.hip): soft taps of one half-width,
 // kf = 2, 4 or 8 >= ceil(2 s) taps, hw = 1, 2 or 4 history words of 64 lags, N <= 1024.
 bool launch_axonal_fwd_arrive(const AxFwd& p, int kf, int hw, hipStream_t stream);
