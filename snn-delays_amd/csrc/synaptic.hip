@@ -1443,33 +1443,79 @@ bool launch_syn_bwd(const SynBwd& a, int block, size_t lds, hipStream_t stream) 
 }
 
 // ---------------------------------------------------------------------------------------
-// Plain multi-step LIF layer: one lane per (b, n), sequential over t.
-__global__ void lif_fwd_kernel(delrec_lif_fwd_args a, Lif k) {
+// Plain multi-step LIF layer: one lane per (b, n), sequential over t. Bound: HBM (12 bytes per
+// element and step forward and backward); a lane's chain hides nothing by itself, so a block of
+// steps is loaded while the block before it runs (past the last step the last one is read
+// again, unused). T250 B256 N512, with one load at a time / so: forward 170 / 75 us (2.3 / 5.2
+// TB/s), backward 179 / 83 us (dx, gy, u).
+constexpr int kLifFwdSteps = 16, kLifBwdSteps = 8;
+
+__global__ void __launch_bounds__(256) lif_fwd_kernel(delrec_lif_fwd_args a, Lif k) {
     const size_t BN = (size_t)a.B * a.N;
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= BN) return;
+    constexpr int S = kLifFwdSteps;
+    float xa[S], xb[S];
+    auto load = [&](int t0, float (&x)[S]) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) x[q] = a.x[(size_t)min(t0 + q, a.T - 1) * BN + e];
+    };
     float v = k.v0;
-    for (int t = 0; t < a.T; ++t) {
-        const size_t o = (size_t)t * BN + e;
-        const float u = lif_charge(k, v, a.x[o]);
-        const float y = lif_fire(k, u);
-        v = lif_reset(k, u, y);
-        a.y[o] = y;
-        a.u[o] = u;
+    auto run = [&](int t0, const float (&x)[S]) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            if (t0 + q >= a.T) break;
+            const size_t o = (size_t)(t0 + q) * BN + e;
+            const float u = lif_charge(k, v, x[q]);
+            const float y = lif_fire(k, u);
+            v = lif_reset(k, u, y);
+            a.y[o] = y;
+            a.u[o] = u;
+        }
+    };
+    load(0, xa);
+    for (int t0 = 0; t0 < a.T; t0 += 2 * S) {
+        if (t0 + S < a.T) load(t0 + S, xb);
+        run(t0, xa);
+        if (t0 + S < a.T) {
+            if (t0 + 2 * S < a.T) load(t0 + 2 * S, xa);
+            run(t0 + S, xb);
+        }
     }
 }
 
-__global__ void lif_bwd_kernel(delrec_lif_bwd_args a, Lif k) {
+__global__ void __launch_bounds__(256) lif_bwd_kernel(delrec_lif_bwd_args a, Lif k) {
     const size_t BN = (size_t)a.B * a.N;
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= BN) return;
+    constexpr int S = kLifBwdSteps;
+    float ga[S], ua[S], gb[S], ub[S];
+    auto load = [&](int t1, float (&g)[S], float (&u)[S]) {   // steps t1, t1 - 1, ..
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            const size_t o = (size_t)max(t1 - q, 0) * BN + e;
+            g[q] = a.gy[o];
+            u[q] = a.u[o];
+        }
+    };
     float lam = 0.0f;
-    for (int t = a.T - 1; t >= 0; --t) {
-        const size_t o = (size_t)t * BN + e;
-        const float u = a.u[o];
-        const float du = lif_backward(k, a.gy[o], u, lif_fire(k, u), lam);
-        lam = k.decay * du;
-        a.dx[o] = lif_dx(k, du);
+    auto run = [&](int t1, const float (&g)[S], const float (&u)[S]) {
+#pragma unroll
+        for (int q = 0; q < S; ++q) {
+            if (t1 - q < 0) break;
+            const float du = lif_backward(k, g[q], u[q], lif_fire(k, u[q]), lam);
+            lam = k.decay * du;
+            a.dx[(size_t)(t1 - q) * BN + e] = lif_dx(k, du);
+        }
+    };
+    load(a.T - 1, ga, ua);
+    for (int t1 = a.T - 1; t1 >= 0; t1 -= 2 * S) {
+        if (t1 - S >= 0) load(t1 - S, gb, ub);
+        run(t1, ga, ua);
+        if (t1 - S >= 0) {
+            if (t1 - 2 * S >= 0) load(t1 - 2 * S, ga, ua);
+            run(t1 - S, gb, ub);
+        }
     }
 }
 
