@@ -482,13 +482,14 @@ void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf
     c.template take<uint4>(packed);                     // gr_lo
     c.template take<uint4>(packed);                     // shifted spikes
     c.template take<int>((size_t)4 * N + 64);           // lag range per column, meta
-    if (hyb_block_on(N, hybrid, offc)) {
+    // (whatever the switches say: a caller may keep the size it was told)
+    if (hybrid && offc > 0 && N <= 1024) {
         const HybBlkShape hb = hyb_block_shape(N, L, bf16, true, 1, 1, 1, (size_t)max_lds_bytes());
         c.template take<uint4>(hb.wq);                  // packed weights
         c.template take<uint4>(hb.oq);                  // packed offsets
         c.template take<int>((size_t)2 * N);            // sources in first-lag order, and its inverse
     }
-    if (syn_lin_on(N, hybrid)) {
+    if (!hybrid && N <= 1024) {
         const SynLinShape sl = syn_lin_shape(N, 2, 1.0f, (size_t)max_lds_bytes());
         c.template take<uint4>(2 * sl.pack);            // packed weights and delays
     }
@@ -1288,7 +1289,7 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     const bool lags_ok = a->d_min >= a->s_uniform - 1.0f;
     HybBlk hbp{};
     HybBlkShape hb{};
-    if (hyb_block_on(N, hybrid, a->off_count)) {
+    if (hybrid && a->off_count > 0 && N <= 1024) {
         hb = hyb_block_shape(N, a->L, a->w_bf16 != 0, true, a->off_count, taps,
                              hyb_block_early(a->d_min, a->s_uniform, lags_ok), (size_t)max_lds_bytes());
         const HybBlkShape room = hyb_block_shape(N, a->L, a->w_bf16 != 0, true, 1, 1, 1, (size_t)max_lds_bytes());
@@ -1297,6 +1298,7 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
         int* ord = cv.take<int>((size_t)2 * N);
         if (!wq || !oq || !ord) return DELREC_ERR_WORKSPACE;
         hbp.wq = wq; hbp.oq = oq; hbp.order = ord; hbp.rank = ord + N;
+        hb.ok = hb.ok && hyb_block_on(N, hybrid, a->off_count);
         if (hb.ok && lags_ok && (KT == 2 || KT == 4) && !hyb_block_pays(N, a->L, a->w_bf16 != 0)) {
             int gs = 0;
             const size_t lds_g = syn_bwd_hyb_g_lds(N, a->L, a->off_count, &gs);
@@ -1309,11 +1311,11 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     // sizes.
     SynLinShape sl{};
     uint4* slp = nullptr;
-    if (syn_lin_on(N, hybrid)) {
+    if (!hybrid && N <= 1024) {
         const SynLinShape room = syn_lin_shape(N, 2, 1.0f, (size_t)max_lds_bytes());
         slp = cv.take<uint4>(2 * room.pack);
         if (!slp) return DELREC_ERR_WORKSPACE;
-        if (!a->s && lay.lds_ring) sl = syn_lin_shape(N, a->L, a->s_uniform, (size_t)max_lds_bytes());
+        if (!a->s && lay.lds_ring && syn_lin_on(N, hybrid)) sl = syn_lin_shape(N, a->L, a->s_uniform, (size_t)max_lds_bytes());
     }
     const bool hybstep = !hb.ok && syn_hybstep(T, B, N, a->L, hybrid && !a->s, a->off_count, taps, lags_ok);
     const bool lagstep = !hb.ok && !sl.ok && !hybstep && syn_lagstep(T, B, N, a->L, taps);
