@@ -283,7 +283,7 @@ def peak_of(w):
 SCAN_SYMBOL = {
     'C1': {'axonal_fwd_scan': 'axonal_fwd_wave_fast', 'axonal_bwd_scan': 'axonal_bwd_tiled_fast'},
     'C2': {'axonal_fwd_scan': 'axonal_fwd_wave_fast', 'axonal_bwd_scan': 'axonal_bwd_tiled_fast'},
-    'C3': {'syn_fwd_scan': 'hyb_fwd_arrive_kernel', 'syn_bwd_scan': 'syn_bwd_hyb_g'},
+    'C3': {'syn_fwd_scan': 'hyb_fwd_arrive_kernel', 'syn_bwd_scan': 'hyb_block_bwd_kernel'},
     'C4': {'syn_fwd_scan': 'lagstep_fwd_sequence', 'syn_bwd_scan': 'lagstep_bwd_sequence'},
     'C5': {'syn_fwd_scan': 'hyb_fwd_arrive_kernel', 'syn_bwd_scan': 'hybstep_bwd_sequence'},
 }
