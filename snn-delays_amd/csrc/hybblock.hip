@@ -23,7 +23,7 @@
 // issue, 4,096 clk at N = 512, is the bound then) and the two exchanges of a step.
 // Measured (scan): T250 B128 N256 sigma 1, 5 offsets, fp32 W 0.65 ms, 2.6 us a step (23.5 ms with
 // the per-tap gather of syn_bwd_kernel); T256 B256 N512 sigma 0, 9 offsets, bf16 W 1.8 ms (2.22 ms
-// with syn_bwd_hyb_g); axonal T250 B256 N512 sigma 1 fp32 W 1.4 ms (8.70 ms with the dense
+// with syn_bwd_hyb_g); axonal T250 B256 N512 sigma 1 fp32 W 1.6 ms (8.70 ms with the dense
 // product streamed per step, axonal_bwd_kernel). A group's whole block taken in one step by its
 // own wave alone: 5.2 ms at N = 512 (one wave per SIMD at a time hides nothing); neurons on the
 // summing waves instead of waves of their own: 2.0 ms (their registers together spill).
