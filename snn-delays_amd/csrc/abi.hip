@@ -449,16 +449,37 @@ int hyb_block_early(float d_min, float s, bool lags_ok) {
     return run <= 2.0 ? 2 : run <= 4.0 ? 4 : run <= 8.0 ? 8 : 16;
 }
 
-// Where every lag is >= 1 and the runs are compiled (KT 2 or 4), syn_bwd_hyb_g sums each step's
-// G whole, in the step, with one barrier; the blocked scan has a second barrier per step and sums
-// the sources that start below lag 4 step by step, but fetches and decodes a connection once per
-// 4 steps. Measured (scan, T96 B64, sigma 0, 5 offsets; syn_bwd_hyb_g / blocked, us):
-//   fp32 W:  N 96 127 / 142   N 160 225 / 220   N 256 478 / 226   N 512 1662 / 680
-//   bf16 W, delays to 30:  N 160 181 / 198   N 256 258 / 214   N 336 407 / 421   N 512 709 / 626
-//   bf16 W, delays to 14:  N 160 181 / 199   N 256 258 / 264   N 336 407 / 494   N 512 708 / 679
-// (the blocked scan works in quarters of 64 receivers: N just past 256 pays for padding).
-bool hyb_block_pays(int N, int L, bool bf16) {
-    return bf16 ? L >= 28 && ((N >= 208 && N <= 256) || N >= 400) : N >= 176;
+// How many sources are near ones (first lag < 4): the caller's count, else what delays spread
+// evenly over the window would give (d + smallest offset < 2 + s).
+int hyb_near_sources(const delrec_syn_bwd_args* a) {
+    if (a->near_known && a->near_lt4 >= 0 && a->near_lt4 <= a->N) return a->near_lt4;
+    const float span = (float)(a->L - 1 - a->off_count) - a->s_uniform;
+    return span <= 2.0f + a->s_uniform ? a->N : (int)((float)a->N * (2.0f + a->s_uniform) / span);
+}
+
+// Whether the blocked scan is the faster one where another compiled form holds the layer: the
+// offset-stacked scan (syn_bwd_hyb_g: every lag >= 1, two or four taps, up to 12 offsets; each
+// step's G whole, in the step, one barrier), else the gather per tap (syn_bwd_hyb). A blocked
+// step has a second barrier and sums the near sources in the step, a receiver run of NT slots
+// each, so the near share decides, and with more than 9 offsets the ring of 32 slots, whose
+// near runs are of 8 slots whatever the lags. Blocked over the other's time (scan, T96 B64) at a
+// near share of 0, 0.1, 0.25, 0.5 and 1:
+//   offset-stacked, 5 or 9 offsets, fp32 W:  N 96 0.86 1.14 1.12 1.14 0.98   N 160 0.64 0.98 0.99 1.07 1.00
+//       N 192 0.50 0.77 0.77 0.81 0.84   N 224 0.48 0.57 0.72 0.80 1.03   N 256 0.55 0.47 0.59 0.72 0.92   N 512 0.35 0.42 0.47 0.59 0.72
+//   bf16 W:  N 192 0.68 1.03 1.00 1.08 1.13   N 224 0.72 0.88 1.05 1.13 1.46   N 256 0.99 0.85 1.01 1.13 1.47
+//       N 320 0.86 1.10 1.29 1.07 1.34   N 400 0.77 0.91 1.07 1.07 1.46   N 512 0.75 0.88 0.97 1.22 1.47
+//       (quarters of 64 receivers: N just past 256 pays for padding; up to 256 the far groups
+//       past the summing waves' first round pay for a second one, 1.10 at N 256 with one near group)
+//   offset-stacked, 10 or 12 offsets:  fp32 N 192 0.62 1.39 1.62 2.25 3.58   bf16 N 512 1.31 2.47 3.42 5.31 9.1
+//   per tap, up to 9 offsets:  0.19 to 0.51 at every share, fp32 and bf16
+//   per tap, ring of 32 slots, fp32 and bf16:  N 64 0.80 0.81 0.81 0.83 0.90   N 224 0.61 0.50 0.70 0.98 1.61
+//       N 400 0.82 0.55 0.78 1.13 1.70   N 512 0.57 0.53 0.74 1.14 1.97
+bool hyb_block_pays(const HybBlkShape& q, int N, int near, bool bf16, bool stacked) {
+    if (!stacked) return q.R <= 16 || 3 * near <= N;
+    if (q.R > 16) return false;
+    if (!bf16) return N >= 176;
+    if (5 * near > N) return false;
+    return N >= 400 || (N >= 208 && N <= 256 && (near == 0 || (N + 15) / 16 - (near + 15) / 16 <= q.nwg));
 }
 
 // The synaptic backward on interpolation tables (synlin.hip): N <= 1024, not under the switches
@@ -1299,11 +1320,14 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
         if (!wq || !oq || !ord) return DELREC_ERR_WORKSPACE;
         hbp.wq = wq; hbp.oq = oq; hbp.order = ord; hbp.rank = ord + N;
         hb.ok = hb.ok && hyb_block_on(N, hybrid, a->off_count);
-        if (hb.ok && lags_ok && (KT == 2 || KT == 4) && !hyb_block_pays(N, a->L, a->w_bf16 != 0)) {
-            int gs = 0;
+        // the other compiled forms: KT 2 or 4, their rings in LDS (the general gather per tap,
+        // at 2.5 times the blocked scan's time or more, is no alternative)
+        int gs = 0;
+        const size_t lds_t = (size_t)((N + 63) / 64 * 64) * lay.RP * sizeof(float);
+        if (hb.ok && N <= 512 && (KT == 2 || KT == 4) && lds_t <= (size_t)max_lds_bytes()) {
             const size_t lds_g = syn_bwd_hyb_g_lds(N, a->L, a->off_count, &gs);
-            const size_t lds_t = (size_t)((N + 63) / 64 * 64) * lay.RP * sizeof(float);
-            if (lds_g && std::max(lds_g, lds_t) <= (size_t)max_lds_bytes()) hb.ok = false;
+            const bool stacked = lags_ok && lds_g && lds_g <= (size_t)max_lds_bytes();
+            hb.ok = hyb_block_pays(hb, N, hyb_near_sources(a), a->w_bf16 != 0, stacked);
         }
     }
     // per-connection delays of one half-width whose tables fit LDS: linear interpolation. The
@@ -1627,6 +1651,8 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
         hbp.KF = taps; hbp.D = hb.Dmax; hbp.room = hb.room; hbp.nwg = hb.nwg; hbp.gy = a->gy; hbp.u = a->u; hbp.base = a->base; hbp.meta = meta;
         hbp.s_uniform = a->s_uniform; hbp.drop = a->drop; hbp.lif = make_lif(a->lif);
         hbp.dx = a->dx; hbp.gr = a->drop ? gr : nullptr; hbp.part = part;
+        if (getenv("DELREC_LOG_PLAN"))
+            fprintf(stderr, "[delrec] hybrid backward: blocked scan, ring of %d slots\n", hb.R);
         launch_hyb_block_pack(hbp, const_cast<uint4*>(hbp.wq), const_cast<uint4*>(hbp.oq),
                               const_cast<int*>(hbp.order), const_cast<int*>(hbp.rank), a->W, a->offsets, a->w_bf16 != 0, s);
         const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
@@ -1674,6 +1700,8 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     const bool hyb_g = hyb_fast && a->d_min >= a->s_uniform - 1.0f && a->off_count > 0 &&
                        getenv_flag_off("DELREC_SYN_BWD_HYB_G") &&
                        launch_syn_bwd_hyb_g(p, a->off_count, (size_t)max_lds_bytes(), s);
+    if (hybrid && getenv("DELREC_LOG_PLAN"))
+        fprintf(stderr, "[delrec] hybrid backward: %s\n", hyb_g ? "offset-stacked scan" : "gather per tap");
     const bool ok = hyb_g || (hyb_fast ? launch_syn_bwd_hyb(p, lay.block, lds_hx, s) : launch_syn_bwd(p, lay.block, lay.lds, s));
     scan_end(timed && ok, s);
     if (!ok) return DELREC_ERR_UNSUPPORTED;

@@ -78,3 +78,35 @@ def test_blocked_backward_with_dropout_and_bias(dev, monkeypatch):
         out.append([xi.grad, bi.grad] + [p.grad for p in layer.parameters()])
     for a, b in zip(*out):
         torch.testing.assert_close(a, b, rtol=1e-4, atol=1e-5 * float(b.abs().max()))
+
+
+# which backward a call takes: sources starting below lag 4 (`near`, a share) are summed step by
+# step in the blocked scan, and more than 9 offsets need its ring of 32 slots, so it gives way to
+# the offset-stacked scan (every lag >= 1) or the gather per tap (sigma 0.5: lags below 1)
+ROUTES = [
+    # N, offsets, bf16 weights, sigma, near share, expected
+    (200, 12, False, 0.0, 0.1, 'offset-stacked'),
+    (200, 5, False, 0.0, 0.5, 'blocked'),
+    (256, 5, True, 0.0, 0.6, 'offset-stacked'),
+    (256, 5, True, 0.0, 0.1, 'blocked'),
+    (256, 9, True, 0.0, 0.03, 'offset-stacked'),    # 15 far groups: one past the summing waves
+    (200, 12, False, 0.5, 0.6, 'gather per tap'),
+    (200, 12, False, 0.5, 0.1, 'blocked'),
+    (200, 5, True, 0.5, 1.0, 'blocked'),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', ROUTES, ids=[f'N{c[0]}K{c[1]}{"bf16" if c[2] else ""}s{c[3]}near{c[4]}' for c in ROUTES])
+def test_backward_form_follows_the_near_share_and_the_offsets(dev, case, monkeypatch, capfd):
+    N, K, bf16, sigma, near, expected = case
+    monkeypatch.setenv('DELREC_LOG_PLAN', '1')
+    g = gen(6)
+    base = 5.0 + torch.rand(N, generator=g) * 25
+    base[:round(near * N)] = torch.rand(round(near * N), generator=g) * 2
+    layer = hybrid_layer(N, torch.randn(N, N, generator=g) / N ** 0.5, base,
+                         torch.randint(K, (N, N), generator=g).float(), dev, bf16=bf16, sigma_init=sigma)
+    x = torch.randn(12, 2, N, generator=g).to(dev).requires_grad_(True)
+    layer(x).sum().backward()
+    torch.cuda.synchronize()
+    assert f'hybrid backward: {expected}' in capfd.readouterr().err
