@@ -333,7 +333,10 @@ enum { DELREC_MAX_SLOTS = 256 };
 int delrec_max_post(const float* x, int32_t n, uint32_t* ticket, void* stream);
 int delrec_max_take(uint32_t ticket, float* out, int32_t timeout_ms);
 
-/* Bytes of scratch the given entry point needs for these sizes and flags. */
+/* Bytes of scratch the given entry point needs for these sizes and flags. The synaptic and
+ * axonal backward keep their fastest scans' operands at the end of it: a smaller workspace that
+ * still holds the rest runs without them, in a slower form, and is DELREC_ERR_WORKSPACE only
+ * past that. */
 int delrec_query_workspace(int32_t kind, int32_t T, int32_t B, int32_t N, int32_t L,
                            int32_t flags, size_t* bytes);
 

@@ -503,7 +503,19 @@ void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf
     c.template take<uint4>(packed);                     // gr_lo
     c.template take<uint4>(packed);                     // shifted spikes
     c.template take<int>((size_t)4 * N + 64);           // lag range per column, meta
-    // (whatever the switches say: a caller may keep the size it was told)
+    if (syn_hybstep(T, B, N, L, hybrid, offc, taps, lags_ok)) {
+        hybstep_ws(c, T, B, N, L, offc, taps, false, bf16);
+    } else if (syn_lagstep(T, B, N, L, taps)) {
+        lagstep_ws(c, T, B, N, L, false);
+    } else {
+        c.template take<float>((size_t)N * lay.NT);     // W^T (fp32 or bf16)
+        c.template take<float>((size_t)N * lay.NT);     // d^T or the offsets^T
+        c.template take<float>((size_t)B * N * lay.RP); // ring when it does not fit LDS
+        c.template take<uint8_t>((size_t)N * lay.NT);   // byte slot offsets (hybrid)
+        c.template take<int>((size_t)N);                // sources in first-lag order (hybrid)
+    }
+    // last, and whatever the switches say (a caller may keep the size it was told): the blocked
+    // and the interpolated scan's operands; a workspace that ends before them takes another form
     if (hybrid && offc > 0 && N <= 1024) {
         const HybBlkShape hb = hyb_block_shape(N, L, bf16, true, 1, 1, 1, (size_t)max_lds_bytes());
         c.template take<uint4>(hb.wq);                  // packed weights
@@ -514,19 +526,6 @@ void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf
         const SynLinShape sl = syn_lin_shape(N, 2, 1.0f, (size_t)max_lds_bytes());
         c.template take<uint4>(2 * sl.pack);            // packed weights and delays
     }
-    if (syn_hybstep(T, B, N, L, hybrid, offc, taps, lags_ok)) {
-        hybstep_ws(c, T, B, N, L, offc, taps, false, bf16);
-        return;
-    }
-    if (syn_lagstep(T, B, N, L, taps)) {
-        lagstep_ws(c, T, B, N, L, false);
-        return;
-    }
-    c.template take<float>((size_t)N * lay.NT);         // W^T (fp32 or bf16)
-    c.template take<float>((size_t)N * lay.NT);         // d^T or the offsets^T
-    c.template take<float>((size_t)B * N * lay.RP);     // ring when it does not fit LDS
-    c.template take<uint8_t>((size_t)N * lay.NT);       // byte slot offsets (hybrid)
-    c.template take<int>((size_t)N);                    // sources in first-lag order (hybrid)
 }
 
 // out[c * op + r] = in[r * n + c] for an (n, n) matrix; output columns r in [n, op) are 0
@@ -1308,18 +1307,26 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     int* meta = cv.take<int>((size_t)4 * N + 64);
     const int taps = lag_taps(hybrid ? a->s_uniform : (a->s ? a->s_max : std::max(a->s_max, a->s_uniform)));
     const bool lags_ok = a->d_min >= a->s_uniform - 1.0f;
+    const bool hybstep = syn_hybstep(T, B, N, a->L, hybrid && !a->s, a->off_count, taps, lags_ok);
+    const bool lagstep = !hybstep && syn_lagstep(T, B, N, a->L, taps);
+    void* wt = nullptr;
+    void* dt = nullptr;
+    float* gring = nullptr;
+    uint8_t* offq = nullptr;
+    int* order = nullptr;
+    if (!lagstep && !hybstep) {
+        wt = cv.take<float>((size_t)N * wlay.NT);
+        dt = cv.take<float>((size_t)N * wlay.NT);
+        gring = cv.take<float>((size_t)B * N * wlay.RP);
+        offq = cv.take<uint8_t>((size_t)N * wlay.NT);
+        order = cv.take<int>((size_t)N);
+        if (!wt || !dt || !gring || !offq || !order) return DELREC_ERR_WORKSPACE;
+    }
     HybBlk hbp{};
     HybBlkShape hb{};
-    if (hybrid && a->off_count > 0 && N <= 1024) {
+    if (hyb_block_on(N, hybrid, a->off_count) && !hybstep && !lagstep) {
         hb = hyb_block_shape(N, a->L, a->w_bf16 != 0, true, a->off_count, taps,
                              hyb_block_early(a->d_min, a->s_uniform, lags_ok), (size_t)max_lds_bytes());
-        const HybBlkShape room = hyb_block_shape(N, a->L, a->w_bf16 != 0, true, 1, 1, 1, (size_t)max_lds_bytes());
-        uint4* wq = cv.take<uint4>(room.wq);
-        uint4* oq = cv.take<uint4>(room.oq);
-        int* ord = cv.take<int>((size_t)2 * N);
-        if (!wq || !oq || !ord) return DELREC_ERR_WORKSPACE;
-        hbp.wq = wq; hbp.oq = oq; hbp.order = ord; hbp.rank = ord + N;
-        hb.ok = hb.ok && hyb_block_on(N, hybrid, a->off_count);
         // the other compiled forms: KT 2 or 4, their rings in LDS (the general gather per tap,
         // at 2.5 times the blocked scan's time or more, is no alternative)
         int gs = 0;
@@ -1329,32 +1336,24 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
             const bool stacked = lags_ok && lds_g && lds_g <= (size_t)max_lds_bytes();
             hb.ok = hyb_block_pays(hb, N, hyb_near_sources(a), a->w_bf16 != 0, stacked);
         }
+        if (hb.ok) {
+            uint4* wq = cv.take<uint4>(hb.wq);
+            uint4* oq = cv.take<uint4>(hb.oq);
+            int* ord = cv.take<int>((size_t)2 * N);
+            hb.ok = wq && oq && ord;
+            hbp.wq = wq; hbp.oq = oq; hbp.order = ord; hbp.rank = ord + N;
+        }
     }
     // per-connection delays of one half-width whose tables fit LDS: linear interpolation. The
-    // entry's own ring (one value per step) must fit too, so that the lag-stacked scan keeps its
-    // sizes.
+    // entry's own ring (one value per step) must fit too.
     SynLinShape sl{};
     uint4* slp = nullptr;
-    if (!hybrid && N <= 1024) {
-        const SynLinShape room = syn_lin_shape(N, 2, 1.0f, (size_t)max_lds_bytes());
-        slp = cv.take<uint4>(2 * room.pack);
-        if (!slp) return DELREC_ERR_WORKSPACE;
-        if (!a->s && lay.lds_ring && syn_lin_on(N, hybrid)) sl = syn_lin_shape(N, a->L, a->s_uniform, (size_t)max_lds_bytes());
-    }
-    const bool hybstep = !hb.ok && syn_hybstep(T, B, N, a->L, hybrid && !a->s, a->off_count, taps, lags_ok);
-    const bool lagstep = !hb.ok && !sl.ok && !hybstep && syn_lagstep(T, B, N, a->L, taps);
-    void* wt = nullptr;
-    void* dt = nullptr;
-    float* gring = nullptr;
-    uint8_t* offq = nullptr;
-    int* order = nullptr;
-    if (!lagstep && !hybstep && !hb.ok && !sl.ok) {
-        wt = cv.take<float>((size_t)N * wlay.NT);
-        dt = cv.take<float>((size_t)N * wlay.NT);
-        gring = cv.take<float>((size_t)B * N * wlay.RP);
-        offq = cv.take<uint8_t>((size_t)N * wlay.NT);
-        order = cv.take<int>((size_t)N);
-        if (!wt || !dt || !gring || !offq || !order) return DELREC_ERR_WORKSPACE;
+    if (syn_lin_on(N, hybrid) && !lagstep && !a->s && lay.lds_ring) {
+        sl = syn_lin_shape(N, a->L, a->s_uniform, (size_t)max_lds_bytes());
+        if (sl.ok) {
+            slp = cv.take<uint4>(2 * sl.pack);
+            sl.ok = slp != nullptr;
+        }
     }
     if (!gr || !part || !lagp || !ahi || !amd || !alo || !yb || !meta) return DELREC_ERR_WORKSPACE;
 
