@@ -157,8 +157,10 @@ typedef struct {
      * can be larger when the source of the smallest base has no connection at off_min.
      * The caller reads them with the window length. A call that breaks either contract
      * (an offset outside [off_min, off_min + off_count), or a source whose taps reach a lag
-     * < 1 in those forms) gets NaN in the outputs that connection or source reaches,
-     * never silently dropped taps. */
+     * < 1 in those forms) gets NaN in the outputs that connection or source reaches (the
+     * backward: in every output), never silently dropped taps. With d_min < s_uniform - 1, or
+     * off_count > 16, the two only pick the backward's fastest scan (blocked, N <= 1024): values
+     * that do not hold cost time, not results. */
     float d_min;
     int32_t off_min;
     int32_t off_count;

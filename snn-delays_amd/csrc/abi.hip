@@ -195,7 +195,7 @@ void axonal_block_ws(C& c, int T, int B, int N) {
     const HybBlkShape q = hyb_block_shape(N, 1, false, false, 1, 1, 1, (size_t)max_lds_bytes());
     c.template take<float>((size_t)T * B * N);
     c.template take<uint4>(q.wq);
-    c.template take<int>((size_t)2 * N);
+    c.template take<int>((size_t)2 * N + 1);
 }
 
 // ------------------------------------------------------------------ synaptic layout ----
@@ -520,7 +520,7 @@ void syn_bwd_ws(C& c, int T, int B, int N, int L, int taps, bool hybrid, bool bf
         const HybBlkShape hb = hyb_block_shape(N, L, bf16, true, 1, 1, 1, (size_t)max_lds_bytes());
         c.template take<uint4>(hb.wq);                  // packed weights
         c.template take<uint4>(hb.oq);                  // packed offsets
-        c.template take<int>((size_t)2 * N);            // sources in first-lag order, and its inverse
+        c.template take<int>((size_t)2 * N + 1);        // sources in first-lag order, its inverse, a flag
     }
     if (!hybrid && N <= 1024) {
         const SynLinShape sl = syn_lin_shape(N, 2, 1.0f, (size_t)max_lds_bytes());
@@ -914,7 +914,7 @@ int delrec_axonal_bwd(const delrec_axonal_bwd_args* a, void* stream) {
     if (hb.ok) {
         gzbuf = cv.take<float>((size_t)T * B * N);
         hwq = cv.take<uint4>(hb.wq);
-        hord = cv.take<int>((size_t)2 * N);
+        hord = cv.take<int>((size_t)2 * N + 1);
         hb.ok = gzbuf && hwq && hord;
     }
     const bool need_gr = a->drop != nullptr || a->lif.decay_input;
@@ -939,10 +939,10 @@ int delrec_axonal_bwd(const delrec_axonal_bwd_args* a, void* stream) {
     if (hb.ok) {
         HybBlk h{};
         h.T = T; h.B = B; h.N = N; h.NCl = hb.NCl; h.Ns = hb.Ns; h.RG = hb.RG; h.KF = (int)std::ceil(2.0f * a->s_uniform);
-        h.D = hb.Dmax; h.room = hb.room; h.nwg = hb.nwg; h.gy = a->gy; h.u = a->u; h.wq = hwq; h.base = a->d;
-        h.order = hord; h.rank = hord + N; h.s_uniform = a->s_uniform; h.drop = a->drop; h.lif = make_lif(a->lif);
+        h.room = hb.room; h.nwg = hb.nwg; h.gy = a->gy; h.u = a->u; h.wq = hwq; h.base = a->d;
+        h.order = hord; h.rank = hord + N; h.wrong = hord + 2 * N; h.s_uniform = a->s_uniform; h.drop = a->drop; h.lif = make_lif(a->lif);
         h.dx = a->dx; h.gr = need_gr ? grbuf : nullptr; h.part = part; h.gz = gzbuf;
-        launch_hyb_block_pack(h, hwq, nullptr, hord, hord + N, a->W, nullptr, a->w_bf16 != 0, s);
+        launch_hyb_block_pack(h, hb, hwq, nullptr, hord, a->W, nullptr, a->w_bf16 != 0, s);
         ok = launch_hyb_block_bwd(h, hb, a->w_bf16 != 0, s);
     } else if (common) {
         const size_t lds_f = ((size_t)2 * lay.NZ + (size_t)(R + kf - 1) * NP) * sizeof(float);
@@ -1339,9 +1339,9 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
         if (hb.ok) {
             uint4* wq = cv.take<uint4>(hb.wq);
             uint4* oq = cv.take<uint4>(hb.oq);
-            int* ord = cv.take<int>((size_t)2 * N);
+            int* ord = cv.take<int>((size_t)2 * N + 1);
             hb.ok = wq && oq && ord;
-            hbp.wq = wq; hbp.oq = oq; hbp.order = ord; hbp.rank = ord + N;
+            hbp.wq = wq; hbp.oq = oq; hbp.order = ord; hbp.rank = ord + N; hbp.wrong = ord + 2 * N;
         }
     }
     // per-connection delays of one half-width whose tables fit LDS: linear interpolation. The
@@ -1645,35 +1645,6 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
         return finish_launch();
     }
 
-    if (hb.ok) {
-        hbp.T = T; hbp.B = B; hbp.N = N; hbp.NCl = hb.NCl; hbp.Ns = hb.Ns; hbp.RG = hb.RG;
-        hbp.KF = taps; hbp.D = hb.Dmax; hbp.room = hb.room; hbp.nwg = hb.nwg; hbp.gy = a->gy; hbp.u = a->u; hbp.base = a->base; hbp.meta = meta;
-        hbp.s_uniform = a->s_uniform; hbp.drop = a->drop; hbp.lif = make_lif(a->lif);
-        hbp.dx = a->dx; hbp.gr = a->drop ? gr : nullptr; hbp.part = part;
-        if (getenv("DELREC_LOG_PLAN"))
-            fprintf(stderr, "[delrec] hybrid backward: blocked scan, ring of %d slots\n", hb.R);
-        launch_hyb_block_pack(hbp, const_cast<uint4*>(hbp.wq), const_cast<uint4*>(hbp.oq),
-                              const_cast<int*>(hbp.order), const_cast<int*>(hbp.rank), a->W, a->offsets, a->w_bf16 != 0, s);
-        const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
-        const bool ok = launch_hyb_block_bwd(hbp, hb, a->w_bf16 != 0, s);
-        scan_end(timed && ok, s);
-        if (!ok) return DELREC_ERR_UNSUPPORTED;
-        return syn_bwd_finish(a, g, gr, part, q.KS, s);
-    }
-
-    if (sl.ok) {
-        SynLin p{};
-        p.T = T; p.B = B; p.N = N; p.L = a->L; p.NC = sl.NC; p.Ns = sl.Ns; p.slices = sl.slices; p.per = sl.per;
-        p.m = sl.m; p.R = sl.R; p.w_bf16 = a->w_bf16; p.gy = a->gy; p.u = a->u; p.wq = slp; p.fq = slp + sl.pack;
-        p.s_uniform = a->s_uniform; p.drop = a->drop; p.lif = make_lif(a->lif);
-        p.dx = a->dx; p.gr = a->drop ? gr : nullptr; p.part = part;
-        const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
-        const bool ok = launch_syn_lin_bwd(p, sl, slp, slp + sl.pack, a->W, a->d, s);
-        scan_end(timed && ok, s);
-        if (!ok) return DELREC_ERR_UNSUPPORTED;
-        return syn_bwd_finish(a, g, gr, part, q.KS, s);
-    }
-
     SynBwd p{};
     p.T = T; p.B = B; p.N = N; p.L = a->L;
     p.R = lay.R; p.RS = lay.RS; p.RP = lay.RP; p.KT = lay.KT; p.NT = lay.NT;
@@ -1685,6 +1656,45 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
     p.s = a->s; p.s_uniform = a->s_uniform;
     p.drop = a->drop; p.lif = make_lif(a->lif);
     p.dx = a->dx; p.gr = gr; p.part = part; p.gring = lay.lds_ring ? nullptr : gring;
+
+    if (hb.ok) {
+        // a smallest delay or an offset count that the device data contradict: NaN outputs where
+        // the header says so (a smallest delay >= s - 1 and up to 16 offsets, which other forms
+        // rely on too), else the general scan in the blocked one's place
+        const bool stated = lags_ok && a->off_count <= 16;
+        hbp.T = T; hbp.B = B; hbp.N = N; hbp.NCl = hb.NCl; hbp.Ns = hb.Ns; hbp.RG = hb.RG;
+        hbp.KF = taps; hbp.room = hb.room; hbp.nwg = hb.nwg; hbp.gy = a->gy; hbp.u = a->u; hbp.base = a->base; hbp.meta = meta;
+        hbp.s_uniform = a->s_uniform; hbp.drop = a->drop; hbp.lif = make_lif(a->lif);
+        hbp.dx = a->dx; hbp.gr = a->drop ? gr : nullptr; hbp.part = part;
+        hbp.wt = stated ? nullptr : wt; hbp.offt = stated ? nullptr : static_cast<int8_t*>(dt);
+        if (getenv("DELREC_LOG_PLAN"))
+            fprintf(stderr, "[delrec] hybrid backward: blocked scan, ring of %d slots\n", hb.R);
+        launch_hyb_block_pack(hbp, hb, const_cast<uint4*>(hbp.wq), const_cast<uint4*>(hbp.oq),
+                              const_cast<int*>(hbp.order), a->W, a->offsets, a->w_bf16 != 0, s);
+        const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
+        const bool ok = launch_hyb_block_bwd(hbp, hb, a->w_bf16 != 0, s);
+        scan_end(timed && ok, s);
+        if (!ok) return DELREC_ERR_UNSUPPORTED;
+        if (!stated) {
+            p.only = hbp.wrong;
+            launch_syn_bwd(p, lay.block, lay.lds, s);
+        }
+        return syn_bwd_finish(a, g, gr, part, q.KS, s);
+    }
+
+    if (sl.ok) {
+        SynLin l{};
+        l.T = T; l.B = B; l.N = N; l.L = a->L; l.NC = sl.NC; l.Ns = sl.Ns; l.slices = sl.slices; l.per = sl.per;
+        l.m = sl.m; l.R = sl.R; l.w_bf16 = a->w_bf16; l.gy = a->gy; l.u = a->u; l.wq = slp; l.fq = slp + sl.pack;
+        l.s_uniform = a->s_uniform; l.drop = a->drop; l.lif = make_lif(a->lif);
+        l.dx = a->dx; l.gr = a->drop ? gr : nullptr; l.part = part;
+        const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
+        const bool ok = launch_syn_lin_bwd(l, sl, slp, slp + sl.pack, a->W, a->d, s);
+        scan_end(timed && ok, s);
+        if (!ok) return DELREC_ERR_UNSUPPORTED;
+        return syn_bwd_finish(a, g, gr, part, q.KS, s);
+    }
+
     const bool timed = scan_begin(DELREC_WS_SYN_BWD, s);
     // room for rows that also mirror the offset span (up to L more slots): the kernel
     // takes the no-wrap form when the span it finds fits

@@ -87,13 +87,17 @@ __device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[4
 }  // namespace
 
 // order[k] = the source with the k-th smallest (first lag, index), rank its inverse. One workgroup, N <= 1024:
-// each thread ranks one source against all keys, four per LDS read.
-__global__ void __launch_bounds__(1024) hyb_block_order_kernel(const float* base, float sv, int N, int* order, int* rank) {
+// each thread ranks one source against all keys, four per LDS read. *wrong: the device data
+// contradict what the caller stated -- the offsets span more than D steps, or a source starts
+// before the lag that early runs of NT slots reach.
+__global__ void __launch_bounds__(1024) hyb_block_order_kernel(const float* base, float sv, int N, const int* meta,
+                                                               int NT, int D, int* order, int* rank, int* wrong) {
     __shared__ __align__(16) int key[1024];
     const int j = threadIdx.x;
     const int kj = j < N ? first_lag(1.0f + base[j], sv) : 0x7fffffff;
     key[j] = kj;
-    __syncthreads();
+    const bool early = __syncthreads_or(meta && j < N && kj + meta[1] < 2 - NT) != 0;
+    if (j == 0) *wrong = meta && (early || meta[2] - meta[1] + 1 > D) ? 1 : 0;
     if (j >= N) return;
     int pos = 0;
     for (int q = 0; q < N; q += 4) {
@@ -108,7 +112,8 @@ __global__ void __launch_bounds__(1024) hyb_block_order_kernel(const float* base
 // The scan's operands in lane order: chunk c of 16 receivers, lane slot js = source order[js],
 //   wq[(c * WV + h) * Ns + js]: the weights of receivers 16 c + 4 h .. (bf16: 8 h ..), WV uint4,
 //   oq[c * Ns + js]: 16 bytes 4 (off - min off);
-// zero past N in either direction.
+// zero past N in either direction. Where the general scan runs in its place: that one's blocked
+// copies (SynBwd::Wt, offt).
 template <bool WBF>
 __global__ void __launch_bounds__(256) hyb_block_pack_kernel(HybBlk p, uint4* wq, uint4* oq, const void* W,
                                                              const int8_t* off) {
@@ -117,6 +122,17 @@ __global__ void __launch_bounds__(256) hyb_block_pack_kernel(HybBlk p, uint4* wq
     const int q = blockIdx.x * 256 + threadIdx.x;
     if (q >= total) return;
     const int c = q / p.Ns, js = q - c * p.Ns;
+    if (p.wt && *p.wrong) {
+        if (c * 16 >= N || js >= N) return;
+        for (int e = 0; e < 16; ++e) {
+            const int i = c * 16 + e;
+            const size_t to = ((size_t)c * N + js) * 16 + e, at = (size_t)i * N + js;
+            if constexpr (WBF) static_cast<uint16_t*>(p.wt)[to] = i < N ? static_cast<const uint16_t*>(W)[at] : 0;
+            else static_cast<uint32_t*>(p.wt)[to] = i < N ? static_cast<const uint32_t*>(W)[at] : 0u;
+            p.offt[to] = i < N ? off[at] : 0;
+        }
+        return;
+    }
     const int j = js < N ? p.order[js] : 0;
     const int omin = off ? p.meta[1] : 0;
     uint32_t w[WV * 4], o[4] = {0, 0, 0, 0};
@@ -154,6 +170,10 @@ __global__ void __launch_bounds__(256) hyb_block_pack_kernel(HybBlk p, uint4* wq
 template <int GPW, int NPL, bool WBF, bool OFF, int R, int PITCH, int NT>
 __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
     extern __shared__ float smem[];
+    // (OFF) what the caller stated does not hold: the general scan, launched behind this one,
+    // takes the call, or every output becomes NaN
+    const bool wrong = OFF && *p.wrong != 0;
+    if (wrong && p.wt) return;
     constexpr int WV = WBF ? 2 : 4;                        // uint4 of W per chunk
     constexpr int CPW = 16 / WV;                           // receivers per uint4 of W
     constexpr uint32_t MB = R * 4 - 1;                     // byte offset within the R slots
@@ -167,7 +187,6 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
     const int ngroups = (N + 15) >> 4;
     const float sv = p.s_uniform;
     const int omin = p.meta ? p.meta[1] : 0;
-    const int D = p.meta ? p.meta[2] - omin + 1 : 1;
     auto lag_of = [&](int j) {                             // (one offset: taps below lag 1 are dropped)
         const int l = first_lag(1.0f + p.base[j], sv) + omin;
         return OFF ? l : max(l, 1);
@@ -175,9 +194,6 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
     // groups in first-lag order: near ones first
     const int glo = tid < ngroups ? lag_of(p.order[tid * 16]) : 0x7fffffff;
     const int nn = __syncthreads_count(glo < 4);
-    // a caller's claims that the device data contradict (offsets past the stated range, a
-    // source that starts earlier than the smallest delay it gave) make every output NaN
-    const bool wrong = OFF && (D > p.D || __syncthreads_or(glo < 2 - NT) != 0);
 
     const int rowsq = NCl * 16 * PITCH + PAD;              // words per quarter
     float* ghist = smem + 4 * rowsq + 64;                  // [RG][Ns], column = source
@@ -651,10 +667,10 @@ HybBlkShape hyb_block_shape(int N, int L, bool bf16, bool offsets, int D, int KF
     return q;
 }
 
-void launch_hyb_block_pack(const HybBlk& p, uint4* wq, uint4* oq, int* order, int* rank, const void* W,
+void launch_hyb_block_pack(const HybBlk& p, const HybBlkShape& q, uint4* wq, uint4* oq, int* order, const void* W,
                            const int8_t* off, bool bf16, hipStream_t s) {
-    hipLaunchKernelGGL(hyb_block_order_kernel, dim3(1), dim3(1024), 0, s, p.base, p.s_uniform, p.N, order,
-                       rank);
+    hipLaunchKernelGGL(hyb_block_order_kernel, dim3(1), dim3(1024), 0, s, p.base, p.s_uniform, p.N, p.meta, q.NT,
+                       q.Dmax, order, order + p.N, order + 2 * p.N);
     const int blocks = (4 * p.NCl * p.Ns + 255) / 256;
     if (bf16) hipLaunchKernelGGL(hyb_block_pack_kernel<true>, dim3(blocks), dim3(256), 0, s, p, wq, oq, W, off);
     else hipLaunchKernelGGL(hyb_block_pack_kernel<false>, dim3(blocks), dim3(256), 0, s, p, wq, oq, W, off);

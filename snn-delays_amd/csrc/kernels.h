@@ -105,6 +105,7 @@ struct SynBwd {
     int ldsf;                   // floats of LDS the hybrid backward was given
     const int* order;           // hybrid: source of each lane slot (first-lag order), or NULL
     const uint8_t* offq;        // blocked (offset - smallest offset) * 4 as bytes (hybrid), or NULL
+    const int* only;            // run only where *only != 0, or NULL (syn_bwd_kernel)
 };
 
 // The synaptic reverse scan on interpolation tables (synlin.hip): one half-width, windows of up to
@@ -143,7 +144,7 @@ struct HybBlkShape {
     size_t lds, wq, oq;         // LDS bytes, uint4 of the packed weights and offsets
 };
 struct HybBlk {
-    int T, B, N, NCl, Ns, RG, KF, D, room, nwg;
+    int T, B, N, NCl, Ns, RG, KF, room, nwg;
     const float* gy;
     const float* u;
     const uint4* wq;
@@ -151,6 +152,9 @@ struct HybBlk {
     const float* base;          // hybrid base, or the axonal delays
     const int* order;           // sources in first-lag order
     const int* rank;            // and its inverse
+    const int* wrong;           // != 0: the stated offset range or smallest delay does not hold
+    void* wt;                   // room for the general scan's blocked W^T, which then takes the
+    int8_t* offt;               // call, and its offsets^T; NULL: NaN outputs instead
     const int* meta;            // meta[1], meta[2] = smallest and largest offset, or NULL
     float s_uniform;
     const float* drop;
@@ -161,7 +165,8 @@ struct HybBlk {
     float* gz;                  // (T,B,N) G, or NULL
 };
 HybBlkShape hyb_block_shape(int N, int L, bool bf16, bool offsets, int D, int KF, int NT, size_t max_lds);
-void launch_hyb_block_pack(const HybBlk& p, uint4* wq, uint4* oq, int* order, int* rank, const void* W,
+// order: 2 N + 1 ints (the order, its inverse, HybBlk::wrong)
+void launch_hyb_block_pack(const HybBlk& p, const HybBlkShape& q, uint4* wq, uint4* oq, int* order, const void* W,
                            const int8_t* off, bool bf16, hipStream_t s);
 bool launch_hyb_block_bwd(const HybBlk& p, const HybBlkShape& q, bool bf16, hipStream_t s);
 

@@ -610,6 +610,7 @@ __global__ void __launch_bounds__(1024) syn_fwd_gather_kernel(SynFwd p) {
 template <int NPT, int KT, bool HYB, int MAXT, bool GRING>
 __global__ void __launch_bounds__(MAXT) syn_bwd_kernel(SynBwd p) {
     extern __shared__ float smem[];
+    if (p.only && *p.only == 0) return;
     constexpr int KA = (HYB && KT > 0) ? KT : 1;        // per-tap accumulators (hybrid, fixed KT)
     const int N = p.N, T = p.T, B = p.B, R = p.R, RP = p.RP;
     const int kt = KT > 0 ? KT : p.KT;                  // KT == 0: the tap count is a runtime value

@@ -110,3 +110,59 @@ def test_backward_form_follows_the_near_share_and_the_offsets(dev, case, monkeyp
     layer(x).sum().backward()
     torch.cuda.synchronize()
     assert f'hybrid backward: {expected}' in capfd.readouterr().err
+
+
+# a smallest delay that is too large but still below s - 1, or an offset count that is too small
+# there (and, above 16 offsets, wherever the lags lie): no form may rely on them, so the
+# gradients are the oracle's. (d_min, off_min, off_count) -> what the call states instead
+MISSTATED = [
+    ((22, 2, 200, (-4.0, 12.0), 4, False, 1.0), lambda d, o, n: (0.0, o, n)),
+    ((22, 2, 48, (-6.0, 12.0), 4, True, 3.0), lambda d, o, n: (1.9, o, n)),
+    ((22, 2, 200, (0.0, 30.0), 11, False, 1.0), lambda d, o, n: (d, o, 5)),
+    ((22, 1, 530, (-2.0, 8.0), 3, False, 1.0), lambda d, o, n: (0.5, o, n)),
+    ((30, 2, 200, (-0.5, 40.0), 16, False, 0.0), lambda d, o, n: (0.0, o, n)),
+]
+
+
+def _state(monkeypatch, change):
+    from delrec.kernels import synaptic_eventdriven as se
+    real = se.hybrid_form
+
+    def form(d_min, s, rng):
+        d, o, n = change(d_min, *rng)
+        return real(d, s, (o, n))
+
+    monkeypatch.setattr(se, 'hybrid_form', form)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case,change', MISSTATED, ids=[f'N{c[0][2]}K{c[0][4]}s{c[0][6]}' for c in MISSTATED])
+def test_blocked_backward_does_not_rely_on_a_misstated_range(dev, case, change, monkeypatch, capfd):
+    _state(monkeypatch, change)
+    monkeypatch.setenv('DELREC_LOG_PLAN', '1')
+    check_case(dev, case)
+    assert 'hybrid backward: blocked' in capfd.readouterr().err
+
+
+# where every lag is said to be >= 1 (and up to 16 offsets), the scans do rely on the stated
+# range: a call that breaks it gets NaN everywhere, never a wrong gradient
+REFUSED = [
+    ((22, 2, 200, (-0.5, 30.0), 4, False, 0.0), lambda d, o, n: (0.0, o, n)),
+    ((22, 2, 256, (0.0, 30.0), 11, False, 0.0), lambda d, o, n: (d, o, 5)),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case,change', REFUSED, ids=['d_min', 'offsets'])
+def test_blocked_backward_refuses_a_broken_range(dev, case, change, monkeypatch, capfd):
+    T, B, N, (lo, hi), K, bf16, sigma = case
+    _state(monkeypatch, change)
+    monkeypatch.setenv('DELREC_LOG_PLAN', '1')
+    g = gen(2)
+    layer = hybrid_layer(N, torch.randn(N, N, generator=g) / N ** 0.5, lo + torch.rand(N, generator=g) * (hi - lo),
+                         torch.randint(K + 1, (N, N), generator=g).float(), dev, bf16=bf16, sigma_init=sigma)
+    x = torch.randn(T, B, N, generator=g).to(dev).requires_grad_(True)
+    layer(x).sum().backward()
+    torch.cuda.synchronize()
+    assert 'hybrid backward: blocked' in capfd.readouterr().err
+    assert bool(x.grad.isnan().all())
