@@ -938,7 +938,7 @@ int delrec_axonal_bwd(const delrec_axonal_bwd_args* a, void* stream) {
     bool ok;
     if (hb.ok) {
         HybBlk h{};
-        h.T = T; h.B = B; h.N = N; h.NCl = hb.NCl; h.Ns = hb.Ns; h.RG = hb.RG; h.KF = (int)std::ceil(2.0f * a->s_uniform);
+        h.T = T; h.B = B; h.N = N; h.L = a->L; h.NCl = hb.NCl; h.Ns = hb.Ns; h.RG = hb.RG; h.KF = (int)std::ceil(2.0f * a->s_uniform);
         h.room = hb.room; h.nwg = hb.nwg; h.gy = a->gy; h.u = a->u; h.wq = hwq; h.base = a->d;
         h.order = hord; h.rank = hord + N; h.wrong = hord + 2 * N; h.s_uniform = a->s_uniform; h.drop = a->drop; h.lif = make_lif(a->lif);
         h.dx = a->dx; h.gr = need_gr ? grbuf : nullptr; h.part = part; h.gz = gzbuf;
@@ -1662,7 +1662,7 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
         // the header says so (a smallest delay >= s - 1 and up to 16 offsets, which other forms
         // rely on too), else the general scan in the blocked one's place
         const bool stated = lags_ok && a->off_count <= 16;
-        hbp.T = T; hbp.B = B; hbp.N = N; hbp.NCl = hb.NCl; hbp.Ns = hb.Ns; hbp.RG = hb.RG;
+        hbp.T = T; hbp.B = B; hbp.N = N; hbp.L = a->L; hbp.NCl = hb.NCl; hbp.Ns = hb.Ns; hbp.RG = hb.RG;
         hbp.KF = taps; hbp.room = hb.room; hbp.nwg = hb.nwg; hbp.gy = a->gy; hbp.u = a->u; hbp.base = a->base; hbp.meta = meta;
         hbp.s_uniform = a->s_uniform; hbp.drop = a->drop; hbp.lif = make_lif(a->lif);
         hbp.dx = a->dx; hbp.gr = a->drop ? gr : nullptr; hbp.part = part;

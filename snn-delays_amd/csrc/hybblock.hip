@@ -346,6 +346,7 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
         const Lif k = p.lif;
         const uint32_t row_bytes = (uint32_t)BN * 4u;
         const float is2 = 1.0f / (sv * sv);
+        const uint32_t lags = (uint32_t)(p.L - 1);         // of the window: 1 .. L - 1
         int jn[NPL], lon[NPL], voff[NPL];
         float m[NPL], cn[NPL], x0[NPL], lam[NPL], dbacc[NPL];
         float* own[NPL];
@@ -429,7 +430,7 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
                 for (int i = 0; i < NPL; ++i)
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        int sl = g1 + min(max(lon[i] + f0 + q, 1), RG - 1) - 1;
+                        int sl = g1 + min(max(lon[i] + f0 + q, 1), RG - 1) - 1;   // (outside the window: unused)
                         sl = sl >= RG ? sl - RG : sl;
                         gv[i][q] = ghist[__umul24(sl, Ns) + max(jn[i], 0)];
                     }
@@ -438,7 +439,7 @@ __global__ void __launch_bounds__(1024) hyb_block_bwd_kernel(HybBlk p) {
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
                         const float h = fmaxf(sv - fabsf(x0[i] + (float)(f0 + q)), 0.0f);
-                        gfs[i] = fmaf(lon[i] + f0 + q >= 1 ? h : 0.0f, gv[i][q], gfs[i]);
+                        gfs[i] = fmaf((uint32_t)(lon[i] + f0 + q - 1) < lags ? h : 0.0f, gv[i][q], gfs[i]);
                     }
             }
 #pragma unroll

@@ -144,7 +144,7 @@ struct HybBlkShape {
     size_t lds, wq, oq;         // LDS bytes, uint4 of the packed weights and offsets
 };
 struct HybBlk {
-    int T, B, N, NCl, Ns, RG, KF, room, nwg;
+    int T, B, N, L, NCl, Ns, RG, KF, room, nwg;
     const float* gy;
     const float* u;
     const uint4* wq;

@@ -5,6 +5,8 @@ one neuron past a wave or a group, two and four neurons per lane, up to 640 and 
 history words, a last partial block of steps, more than 64 arrivals in a step, one step, and the
 neuron's options. Tolerances: ``tests/helpers.py``."""
 
+import ctypes
+
 import pytest
 import torch
 
@@ -50,3 +52,43 @@ def test_wide_axonal_repeats_bit_for_bit(dev):
         out.append([y.detach(), xs.grad, Ws.grad, ds.grad])
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+def _abi(dev, T, B, N, L, sigma, per_source, g, d):
+    """Forward and backward through the C ABI; ``per_source``: the half-width as a vector, which
+    takes the dense scans."""
+    from delrec import _lib
+    lib = _lib.load()
+    x, gy = (torch.randn(T, B, N, generator=g) * 1.2 + 0.3).to(dev), torch.randn(T, B, N, generator=g).to(dev)
+    W, d = (torch.randn(N, N, generator=g) / N ** 0.5).to(dev), d.to(dev)
+    s = torch.full((N,), 1.0 + sigma, device=dev) if per_source else None
+    lif = _lib.make_lif(2.0, 1.0, 0.0, False, False, 1, 1.0, 2.0)
+    y, u, z, dx = (torch.empty(T, B, N, device=dev) for _ in range(4))
+    bits = torch.empty(B, (T + 31) // 32, N, device=dev, dtype=torch.int32)
+    dW, db, dd = torch.empty(N, N, device=dev), torch.empty(N, device=dev), torch.empty(N, device=dev)
+    ws = [_lib.workspace(k, T, B, N, L, 0, dev) for k in (_lib.WS_AXONAL_FWD, _lib.WS_AXONAL_BWD)]
+    both = dict(T=T, B=B, N=N, L=L, W=_lib.ptr(W), w_bf16=0, d=_lib.ptr(d), s=_lib.ptr(s), s_uniform=1.0 + sigma,
+                drop=None, lif=lif, u=_lib.ptr(u), z=_lib.ptr(z), bits=_lib.ptr(bits))
+    fwd = _lib.AxonalFwdArgs(x=_lib.ptr(x), bias=None, taps=0, y=_lib.ptr(y), rec=None, workspace=_lib.ptr(ws[0]),
+                             workspace_bytes=ws[0].numel(), **both)
+    bwd = _lib.AxonalBwdArgs(gy=_lib.ptr(gy), mode=_lib.DELREC_BWD_SOFT, lag=None, dx=_lib.ptr(dx), dW=_lib.ptr(dW),
+                             db=_lib.ptr(db), dd=_lib.ptr(dd), ds=None, workspace=_lib.ptr(ws[1]),
+                             workspace_bytes=ws[1].numel(), **both)
+    assert lib.delrec_axonal_fwd(ctypes.byref(fwd), _lib.stream_of(x)) == 0
+    assert lib.delrec_axonal_bwd(ctypes.byref(bwd), _lib.stream_of(x)) == 0
+    torch.cuda.synchronize()
+    return y, {'dx': dx, 'dW': dW, 'db': db, 'dd': dd}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('sigma', [0.0, 1.0, 3.0])
+def test_wide_axonal_window_cuts_the_taps(dev, sigma):
+    """Delays past the window L: taps at lags 1 .. L - 1 only, as in the dense scans (the same
+    sums in another order: 1e-5 of the largest value)."""
+    T, B, N, L = 40, 2, 300, 12
+    d = torch.rand(N, generator=gen(5)) * 24.0 - 1.0
+    y, got = _abi(dev, T, B, N, L, sigma, False, gen(3), d)
+    yd, dense = _abi(dev, T, B, N, L, sigma, True, gen(3), d)
+    assert torch.equal(y, yd)
+    for k in got:
+        torch.testing.assert_close(got[k], dense[k], rtol=1e-4, atol=1e-5 * float(dense[k].abs().max()), msg=k)
