@@ -183,9 +183,13 @@ void axonal_bwd_ws(C& c, int T, int B, int N, const AxLayout& lay) {
     if (lay.res) c.template take<float>((size_t)T * B * N);                         // gz
 }
 
+// The scans past 256 neurons that serve one half-width (axwide.hip, hybblock.hip) address a step
+// with 32-bit byte offsets, past whose range the lanes without a neuron point: below 2 GiB a step
+bool axonal_step_fits(int B, int N) { return (size_t)B * N * sizeof(float) <= (size_t)0x7fffffc0; }
+
 // The streamed sizes' blocked reverse scan (hybblock.hip, no offsets): soft taps of one half-width
-HybBlkShape axonal_block(int N, int L, bool bf16, float s_uniform, bool per_source) {
-    if (per_source || !(s_uniform > 0.0f) || N <= 256) return HybBlkShape{};
+HybBlkShape axonal_block(int B, int N, int L, bool bf16, float s_uniform, bool per_source) {
+    if (per_source || !(s_uniform > 0.0f) || N <= 256 || !axonal_step_fits(B, N)) return HybBlkShape{};
     return hyb_block_shape(N, L, bf16, false, 1, (int)std::ceil(2.0f * s_uniform), 1, (size_t)max_lds_bytes());
 }
 
@@ -855,7 +859,7 @@ int delrec_axonal_fwd(const delrec_axonal_fwd_args* a, void* stream) {
     const bool timed = scan_begin(DELREC_WS_AXONAL_FWD, s);
     bool ok;
     const float span_f = ceilf(2.0f * a->s_uniform);
-    if (!lay.res && a->taps == DELREC_TAPS_SOFT && !a->s && span_f >= 1.0f && span_f <= 8.0f) {
+    if (!lay.res && a->taps == DELREC_TAPS_SOFT && !a->s && span_f >= 1.0f && span_f <= 8.0f && axonal_step_fits(a->B, a->N)) {
         // N > 256, a uniform half-width: arriving spikes only (T250 B256 N512 sigma 1 at 3.4 %
         // firing: 0.66 ms against 7.99 ms for the dense product streamed from L2)
         ok = launch_axonal_fwd_arrive(p, span_f <= 2.0f ? 2 : span_f <= 4.0f ? 4 : 8, lay.hw, s);
@@ -907,7 +911,7 @@ int delrec_axonal_bwd(const delrec_axonal_bwd_args* a, void* stream) {
     float* gzbuf = lay.res ? cv.take<float>((size_t)T * B * N) : nullptr;
     if (!part || !grbuf || !gemm_part || (lay.res && !gzbuf)) return DELREC_ERR_WORKSPACE;
     // the blocked scan where its buffers are there too (a caller's scratch may end before them)
-    HybBlkShape hb = a->mode == DELREC_BWD_SOFT ? axonal_block(N, a->L, a->w_bf16 != 0, a->s_uniform, a->s != nullptr)
+    HybBlkShape hb = a->mode == DELREC_BWD_SOFT ? axonal_block(B, N, a->L, a->w_bf16 != 0, a->s_uniform, a->s != nullptr)
                                                 : HybBlkShape{};
     uint4* hwq = nullptr;
     int* hord = nullptr;

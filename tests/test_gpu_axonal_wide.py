@@ -92,3 +92,36 @@ def test_wide_axonal_window_cuts_the_taps(dev, sigma):
     assert torch.equal(y, yd)
     for k in got:
         torch.testing.assert_close(got[k], dense[k], rtol=1e-4, atol=1e-5 * float(dense[k].abs().max()), msg=k)
+
+
+@pytest.mark.gpu
+def test_wide_axonal_steps_past_4_gib(dev):
+    """A (B, N) step of more than 4 GiB: past the 32-bit offsets of the scans above. With one step
+    and no spike before it, u = x, y = [x >= 1] and dx = gy sg(x - 1)."""
+    from delrec import _lib
+    lib = _lib.load()
+    B, N, L = 3_600_000, 300, 8
+    print(f'B={B} N={N}: {B * N * 4 / 2 ** 30:.2f} GiB a step', flush=True)
+    g = torch.Generator(dev).manual_seed(1)
+    x = torch.randn(1, B, N, generator=g, device=dev)
+    W, d = torch.randn(N, N, generator=g, device=dev), torch.rand(N, generator=g, device=dev) * 4
+    y, u, z = (torch.full_like(x, 7.0) for _ in range(3))
+    bits = torch.empty(B, 1, N, device=dev, dtype=torch.int32)
+    lif = _lib.make_lif(2.0, 1.0, 0.0, False, False, 1, 1.0, 2.0)
+    both = dict(T=1, B=B, N=N, L=L, W=_lib.ptr(W), w_bf16=0, d=_lib.ptr(d), s=None, s_uniform=1.5, drop=None, lif=lif,
+                u=_lib.ptr(u), bits=_lib.ptr(bits))
+    ws = _lib.workspace(_lib.WS_AXONAL_FWD, 1, B, N, L, 0, dev)
+    fwd = _lib.AxonalFwdArgs(x=_lib.ptr(x), bias=None, taps=0, y=_lib.ptr(y), rec=None, z=_lib.ptr(z),
+                             workspace=_lib.ptr(ws), workspace_bytes=ws.numel(), **both)
+    assert lib.delrec_axonal_fwd(ctypes.byref(fwd), _lib.stream_of(x)) == 0
+    assert torch.equal(u, x) and torch.equal(y, (x >= 1).float()) and float(z.abs().max()) == 0
+    del ws, z
+    gy = y.add_(0.5)
+    dx = torch.full_like(x, 7.0)
+    ws = _lib.workspace(_lib.WS_AXONAL_BWD, 1, B, N, L, 0, dev)
+    bwd = _lib.AxonalBwdArgs(gy=_lib.ptr(gy), z=None, mode=_lib.DELREC_BWD_SOFT, lag=None, dx=_lib.ptr(dx), dW=None,
+                             db=None, dd=None, ds=None, workspace=_lib.ptr(ws), workspace_bytes=ws.numel(), **both)
+    assert lib.delrec_axonal_bwd(ctypes.byref(bwd), _lib.stream_of(x)) == 0
+    # the surrogate's alpha / 2 / (1 + (pi / 2 alpha (u - 1))^2) at alpha = 2
+    ref = gy.div_(x.sub_(1.0).mul_(torch.pi).square_().add_(1.0))
+    assert float(dx.sub_(ref).abs_().max()) < 1e-5
