@@ -48,11 +48,12 @@ __global__ void __launch_bounds__(256) syn_lin_pack_kernel(SynLin p, uint4* wq, 
             fr = 0;
             n += 1;
         }
-        if (n < -m - 1) {                                  // every lag below 1
+        if (n < -m - 1 || dv != dv) {                      // no lag of positive weight: times 0
             n = 0;
-            wv = wv != wv ? wv : 0.0f;
+            fr = 0;
+            wv *= 0.0f;
         }
-        if (dv != dv || n > p.L) {                         // no such delay in the stated window
+        if (n > p.L) {                                     // no such delay in the stated window
             n = 0;
             wv = __builtin_nanf("");
         }

@@ -76,3 +76,36 @@ def test_interpolated_backward_matches_oracle(dev, case):
     plain = drop is None
     check_grads(got, g64, gref, 2e-2 if bf16 else 1e-4, 1e-5, eps=grad_eps(bf16),
                 budget=syn_budget(g64['x'], y.detach().cpu(), d, sigma, W=W) if plain else None)
+
+
+@pytest.mark.gpu
+def test_interpolated_backward_on_delays_and_weights_that_are_no_numbers(dev, monkeypatch):
+    """A NaN delay has no lag of positive weight, and a connection without one is its weight times
+    0 (an infinite weight: NaN in its source's column), as in the gather per tap."""
+    from delrec import _lib
+    from delrec.kernels.synaptic_eventdriven import syn_backward, syn_forward
+    T, B, N, sigma = 19, 2, 48, 1.0
+    g = gen(3)
+    x, gy = (torch.randn(T, B, N, generator=g).to(dev) for _ in range(2))
+    W, d = (torch.randn(N, N, generator=g) / N ** 0.5).to(dev), (torch.rand(N, N, generator=g) * 9).to(dev)
+    lif = _lib.make_lif(2.0, 1.0, 0.0, False, False, 1, 1.0, 2.0)
+    y, u, bits, L, _, _, s_max, _ = syn_forward(x, W, d, None, None, None, 1 + sigma, d, None, None, lif)
+    W, d = W.clone(), d.clone()
+    d[3, 5] = float('nan')
+
+    def both():
+        out = []
+        for switch in ('1', '0'):
+            monkeypatch.setenv('DELREC_SYN_LIN', switch)
+            out.append(syn_backward(gy, u, y, bits, W, 0, d, None, None, None, 1 + sigma, s_max, None, lif, L,
+                                    False, False, False, False)[0])
+        return out
+
+    got, ref = both()
+    assert not torch.equal(got, ref), 'the tables and the gather sum in another order'
+    assert bool(ref.isfinite().all())
+    torch.testing.assert_close(got, ref, rtol=1e-4, atol=1e-5)
+    W[7, 9], d[7, 9] = float('inf'), -30.0
+    for dx in both():
+        assert bool(dx[:, :, 9].isnan().all())
+        assert bool(dx[-1, :, :9].isfinite().all()) and bool(dx[-1, :, 10:].isfinite().all())
