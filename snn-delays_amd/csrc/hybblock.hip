@@ -49,7 +49,8 @@ __device__ __forceinline__ int first_lag(float c, float s) {
 
 // acc[n] += sum over q < 4 of w[q] * (g[n] of lane E + q of the lane's row of 16): the broadcast is
 // an operand modifier of the multiply-add (the compiler makes it a move of its own). The s_nop
-// covers the two wait states a row-modified operand needs after a vector write.
+// covers the two wait states a row-modified operand needs after a vector write; the sums are
+// written before the last operand is read, so they share no register with one (&).
 template <int E>
 __device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[1], float (&acc)[1]) {
     asm("s_nop 1\n\t"
@@ -57,7 +58,7 @@ __device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[1
         "v_fmac_f32_dpp %0, %1, %3 row_newbcast:%7 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f32_dpp %0, %1, %4 row_newbcast:%8 row_mask:0xf bank_mask:0xf\n\t"
         "v_fmac_f32_dpp %0, %1, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf"
-        : "+v"(acc[0])
+        : "+&v"(acc[0])
         : "v"(g[0]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(E), "n"(E + 1), "n"(E + 2), "n"(E + 3));
 }
 
@@ -67,7 +68,7 @@ __device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[1
 template <int E>
 __device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[2], float (&acc)[2]) {
     asm("s_nop 1\n\t" DELREC_FMAC2("%4", "%8") DELREC_FMAC2("%5", "%9") DELREC_FMAC2("%6", "%10") DELREC_FMAC2("%7", "%11")
-        : "+v"(acc[0]), "+v"(acc[1])
+        : "+&v"(acc[0]), "+&v"(acc[1])
         : "v"(g[0]), "v"(g[1]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(E), "n"(E + 1), "n"(E + 2), "n"(E + 3));
 }
 
@@ -79,7 +80,7 @@ __device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[2
 template <int E>
 __device__ __forceinline__ void add_rows(const float (&w)[4], const float (&g)[4], float (&acc)[4]) {
     asm("s_nop 1\n\t" DELREC_FMAC4("%8", "%12") DELREC_FMAC4("%9", "%13") DELREC_FMAC4("%10", "%14") DELREC_FMAC4("%11", "%15")
-        : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3])
+        : "+&v"(acc[0]), "+&v"(acc[1]), "+&v"(acc[2]), "+&v"(acc[3])
         : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "v"(w[0]), "v"(w[1]), "v"(w[2]), "v"(w[3]), "n"(E), "n"(E + 1),
           "n"(E + 2), "n"(E + 3));
 }

@@ -125,3 +125,18 @@ def test_synaptic_scan_form_follows_the_taps_per_connection():
         wide = size(kind, 47, 0, _lib.lag_taps(5.0))         # synaptic, sigma 4
         narrow = size(kind, 66, 2, _lib.lag_taps(1.0))       # hybrid, sigma 0
         assert wide >= planes > narrow
+
+
+def test_assembly_of_several_instructions_writes_no_register_it_still_reads():
+    """An asm statement of several instructions that reads and writes an operand marks it
+    early-clobber ("+&v"): the compiler may otherwise give an input of equal value, read by a
+    later instruction, the same register."""
+    import re
+    from delrec import _build
+    found = 0
+    for src in sorted(_build.CSRC.glob('*.hip')) + sorted(_build.CSRC.glob('*.h')):
+        for stmt in re.findall(r'\basm(?: volatile)?\((.*?)\);', src.read_text(), re.S):
+            if '"+' in stmt and ('\\n' in stmt or 'DELREC_FMAC' in stmt):
+                found += 1
+                assert not re.search(r'"\+v"', stmt), f'{src.name}: {stmt[:80]}'
+    assert found == 3
