@@ -7,8 +7,12 @@
 // lane; nothing is done for silent sources. Per step: the arrivals listed by the step before
 // are walked in a fixed order, eight rows of W^T in flight ahead of the multiply-adds; then the
 // neurons, and each wave's list of the sources arriving next. One barrier per step.
-// Bound: the L2 latency of the first rows and the exchange, then the rows' bytes
-// (N = 512 at 3.4 % firing: 17 rows of 2 KB a step).
+// Bound: at a few percent firing the L2 latency of the first rows and the exchange, then the rows'
+// bytes (N = 512 at 3.4 %: 17 rows of 2 KB a step); past that the multiply-adds' issue, KF to an
+// arrival and wave. Measured (scan, T96 B64, N 512, delays to 25; a readlane before each
+// multiply-add / the row broadcast of add_pair): 3 % firing, sigma 1 249 / 198 us, sigma 3
+// 341 / 242 us; 80 % firing, sigma 1 2.57 / 1.63 ms, sigma 3 4.14 / 2.19 ms. The dense product
+// (axonal_fwd_kernel) takes 3.08 ms whatever the firing.
 #include <algorithm>
 
 #include "common.h"
@@ -17,9 +21,42 @@
 namespace delrec {
 
 namespace {
-constexpr int kRows = 8;        // rows of W^T in flight
+constexpr int kRows = 8;        // rows of W^T in flight (two such blocks: the lanes of a row of 16)
 constexpr int kWaves = 16;
 constexpr int kAhead = 4;       // steps of x loaded together
+
+// pend[f] += h[f] of lane E of the lane's row of 16 times x0, then of lane E + 1 times x1, ..: the
+// broadcast is an operand modifier of the multiply-add (the compiler makes it a move of its
+// own; from a scalar register, a readlane goes before each). The s_nop covers the two wait
+// states a row-modified operand needs after a vector write; the sums are written before the
+// last operand is read, so they share no register with one (&).
+#define DELREC_AXF(P, H, X, E) "v_fmac_f32_dpp %" P ", %" H ", %" X " row_newbcast:%" E " row_mask:0xf bank_mask:0xf\n\t"
+#define DELREC_AXF2(X, E) DELREC_AXF("0", "2", X, E) DELREC_AXF("1", "3", X, E)
+#define DELREC_AXF4(X, E) \
+    DELREC_AXF("0", "4", X, E) DELREC_AXF("1", "5", X, E) DELREC_AXF("2", "6", X, E) DELREC_AXF("3", "7", X, E)
+#define DELREC_AXF8(X, E)                                                                                         \
+    DELREC_AXF("0", "8", X, E) DELREC_AXF("1", "9", X, E) DELREC_AXF("2", "10", X, E) DELREC_AXF("3", "11", X, E) \
+    DELREC_AXF("4", "12", X, E) DELREC_AXF("5", "13", X, E) DELREC_AXF("6", "14", X, E) DELREC_AXF("7", "15", X, E)
+
+template <int E>
+__device__ __forceinline__ void add_pair(float x0, float x1, const float (&h)[2], float (&p)[2]) {
+    asm("s_nop 1\n\t" DELREC_AXF2("4", "6") DELREC_AXF2("5", "7")
+        : "+&v"(p[0]), "+&v"(p[1])
+        : "v"(h[0]), "v"(h[1]), "v"(x0), "v"(x1), "n"(E), "n"(E + 1));
+}
+template <int E>
+__device__ __forceinline__ void add_pair(float x0, float x1, const float (&h)[4], float (&p)[4]) {
+    asm("s_nop 1\n\t" DELREC_AXF4("8", "10") DELREC_AXF4("9", "11")
+        : "+&v"(p[0]), "+&v"(p[1]), "+&v"(p[2]), "+&v"(p[3])
+        : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(x0), "v"(x1), "n"(E), "n"(E + 1));
+}
+template <int E>
+__device__ __forceinline__ void add_pair(float x0, float x1, const float (&h)[8], float (&p)[8]) {
+    asm("s_nop 1\n\t" DELREC_AXF8("16", "18") DELREC_AXF8("17", "19")
+        : "+&v"(p[0]), "+&v"(p[1]), "+&v"(p[2]), "+&v"(p[3]), "+&v"(p[4]), "+&v"(p[5]), "+&v"(p[6]), "+&v"(p[7])
+        : "v"(h[0]), "v"(h[1]), "v"(h[2]), "v"(h[3]), "v"(h[4]), "v"(h[5]), "v"(h[6]), "v"(h[7]), "v"(x0), "v"(x1),
+          "n"(E), "n"(E + 1));
+}
 }  // namespace
 
 // LDS: tap weights [KF][threads], arrival lists [2][16 waves][64], their lengths [2][16]
@@ -115,20 +152,22 @@ __global__ void __launch_bounds__(1024) axonal_fwd_arrive_kernel(AxFwd p) {
                     x[q] = WBF ? bf16_to_f32(raw_buffer_load_u16(rw, wv, so, 0)) : raw_buffer_load_f32(rw, wv, so, 0);
                 }
             };
-            auto add = [&](int q0, const float (&x)[kRows]) {
-#pragma unroll
-                for (int q = 0; q < kRows; ++q)
-#pragma unroll
-                    for (int f = 0; f < KF; ++f)
-                        pend[f] = fmaf(x[q], __int_as_float(__builtin_amdgcn_readlane(__float_as_int(hs[f]), (q0 + q) & 63)), pend[f]);
-            };
             rows(0, wa);
             for (int q0 = 0; q0 < n; q0 += 2 * kRows) {
+                float hr[KF];                              // lane E of every row of 16: arrival q0 + E's weights
+#pragma unroll
+                for (int f = 0; f < KF; ++f) hr[f] = __shfl(hs[f], q0 + (lane & 15));
                 if (q0 + kRows < n) rows(q0 + kRows, wb);
-                add(q0, wa);
+                add_pair<0>(wa[0], wa[1], hr, pend);
+                add_pair<2>(wa[2], wa[3], hr, pend);
+                add_pair<4>(wa[4], wa[5], hr, pend);
+                add_pair<6>(wa[6], wa[7], hr, pend);
                 if (q0 + kRows < n) {
                     if (q0 + 2 * kRows < n) rows(q0 + 2 * kRows, wa);
-                    add(q0 + kRows, wb);
+                    add_pair<8>(wb[0], wb[1], hr, pend);
+                    add_pair<10>(wb[2], wb[3], hr, pend);
+                    add_pair<12>(wb[4], wb[5], hr, pend);
+                    add_pair<14>(wb[6], wb[7], hr, pend);
                 }
             }
         }

@@ -54,13 +54,15 @@ def test_wide_axonal_repeats_bit_for_bit(dev):
         assert torch.equal(a, b)
 
 
-def _abi(dev, T, B, N, L, sigma, per_source, g, d):
+def _abi(dev, T, B, N, L, sigma, per_source, g, d, drive=0.3, grid=0):
     """Forward and backward through the C ABI; ``per_source``: the half-width as a vector, which
-    takes the dense scans."""
+    takes the dense scans. ``drive``: the input's mean; ``grid``: W on multiples of 1 / grid."""
     from delrec import _lib
     lib = _lib.load()
-    x, gy = (torch.randn(T, B, N, generator=g) * 1.2 + 0.3).to(dev), torch.randn(T, B, N, generator=g).to(dev)
+    x, gy = (torch.randn(T, B, N, generator=g) * 1.2 + drive).to(dev), torch.randn(T, B, N, generator=g).to(dev)
     W, d = (torch.randn(N, N, generator=g) / N ** 0.5).to(dev), d.to(dev)
+    if grid:
+        W, x = (W * grid).round() / grid, (x * grid).round() / grid
     s = torch.full((N,), 1.0 + sigma, device=dev) if per_source else None
     lif = _lib.make_lif(2.0, 1.0, 0.0, False, False, 1, 1.0, 2.0)
     y, u, z, dx = (torch.empty(T, B, N, device=dev) for _ in range(4))
@@ -92,6 +94,21 @@ def test_wide_axonal_window_cuts_the_taps(dev, sigma):
     assert torch.equal(y, yd)
     for k in got:
         torch.testing.assert_close(got[k], dense[k], rtol=1e-4, atol=1e-5 * float(dense[k].abs().max()), msg=k)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('sigma', [0.0, 1.0, 3.0])
+@pytest.mark.parametrize('drive', [0.3, 4.0])
+def test_wide_axonal_arrivals_at_dense_firing(dev, sigma, drive):
+    """From a few arrivals a step to most sources at once (several rounds of 64, remainders of 16
+    and 8). With dyadic weights, inputs and delays the recurrent sums are exact in any order, so
+    the spikes are the dense scan's."""
+    T, B, N, L = 50, 2, 330, 30
+    d = (torch.floor(torch.rand(N, generator=gen(5)) * 20 * 16) + 0.5) / 16
+    y, _ = _abi(dev, T, B, N, L, sigma, False, gen(3), d, drive, 4096)
+    yd, _ = _abi(dev, T, B, N, L, sigma, True, gen(3), d, drive, 4096)
+    assert torch.equal(y, yd)
+    assert float(y.mean()) > (0.6 if drive > 1 else 0.05)
 
 
 @pytest.mark.gpu
