@@ -1724,14 +1724,14 @@ int delrec_syn_bwd(const delrec_syn_bwd_args* a, void* stream) {
 int delrec_lif_fwd(const delrec_lif_fwd_args* a, void* stream) {
     if (!a || a->T <= 0 || a->B <= 0 || a->N <= 0 || !a->x || !a->y || !a->u || !lif_ok(a->lif))
         return DELREC_ERR_ARG;
-    launch_lif(true, a, nullptr, make_lif(a->lif), static_cast<hipStream_t>(stream));
+    launch_lif(true, a, nullptr, make_lif(a->lif), num_cus(), static_cast<hipStream_t>(stream));
     return finish_launch();
 }
 
 int delrec_lif_bwd(const delrec_lif_bwd_args* a, void* stream) {
     if (!a || a->T <= 0 || a->B <= 0 || a->N <= 0 || !a->gy || !a->u || !a->dx || !lif_ok(a->lif))
         return DELREC_ERR_ARG;
-    launch_lif(false, nullptr, a, make_lif(a->lif), static_cast<hipStream_t>(stream));
+    launch_lif(false, nullptr, a, make_lif(a->lif), num_cus(), static_cast<hipStream_t>(stream));
     return finish_launch();
 }
 

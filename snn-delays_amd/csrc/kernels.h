@@ -578,7 +578,7 @@ const int* lag_bf16_cls(const LagBf16& a);
 void launch_lag_finish(const LagGemm& a, float* dW, float* dd, float* ds, hipStream_t stream);
 
 void launch_lif(bool fwd, const delrec_lif_fwd_args* fa, const delrec_lif_bwd_args* ba,
-                const Lif& k, hipStream_t stream);
+                const Lif& k, int cus, hipStream_t stream);
 void launch_delay_grad(const float* C, const float* W, const float* d, float sigma, int N,
                        int Lm, float* dd, hipStream_t stream);
 

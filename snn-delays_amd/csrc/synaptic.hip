@@ -1445,17 +1445,17 @@ bool launch_syn_bwd(const SynBwd& a, int block, size_t lds, hipStream_t stream) 
 
 // ---------------------------------------------------------------------------------------
 // Plain multi-step LIF layer: one lane per (b, n), sequential over t. Bound: HBM (12 bytes per
-// element and step forward and backward); a lane's chain hides nothing by itself, so a block of
-// steps is loaded while the block before it runs (past the last step the last one is read
-// again, unused). T250 B256 N512, with one load at a time / so: forward 170 / 75 us (2.3 / 5.2
-// TB/s), backward 179 / 83 us (dx, gy, u).
+// element and step forward and backward). S > 1: a lane's chain hides nothing by itself, so
+// where few waves share a CU a block of S steps is loaded while the block before it runs (past
+// the last step the last one is read again, unused). T250 B256 N512, with one load at a time /
+// so: forward 176 / 82 us (2.2 / 4.8 TB/s), backward 168 / 76 us (dx, gy, u).
 constexpr int kLifFwdSteps = 16, kLifBwdSteps = 8;
 
+template <int S>
 __global__ void __launch_bounds__(256) lif_fwd_kernel(delrec_lif_fwd_args a, Lif k) {
     const size_t BN = (size_t)a.B * a.N;
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= BN) return;
-    constexpr int S = kLifFwdSteps;
     float xa[S], xb[S];
     auto load = [&](int t0, float (&x)[S]) {
 #pragma unroll
@@ -1474,6 +1474,13 @@ __global__ void __launch_bounds__(256) lif_fwd_kernel(delrec_lif_fwd_args a, Lif
             a.u[o] = u;
         }
     };
+    if constexpr (S == 1) {
+        for (int t = 0; t < a.T; ++t) {
+            load(t, xa);
+            run(t, xa);
+        }
+        return;
+    }
     load(0, xa);
     for (int t0 = 0; t0 < a.T; t0 += 2 * S) {
         if (t0 + S < a.T) load(t0 + S, xb);
@@ -1485,11 +1492,11 @@ __global__ void __launch_bounds__(256) lif_fwd_kernel(delrec_lif_fwd_args a, Lif
     }
 }
 
+template <int S>
 __global__ void __launch_bounds__(256) lif_bwd_kernel(delrec_lif_bwd_args a, Lif k) {
     const size_t BN = (size_t)a.B * a.N;
     const size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= BN) return;
-    constexpr int S = kLifBwdSteps;
     float ga[S], ua[S], gb[S], ub[S];
     auto load = [&](int t1, float (&g)[S], float (&u)[S]) {   // steps t1, t1 - 1, ..
 #pragma unroll
@@ -1509,6 +1516,13 @@ __global__ void __launch_bounds__(256) lif_bwd_kernel(delrec_lif_bwd_args a, Lif
             a.dx[(size_t)(t1 - q) * BN + e] = lif_dx(k, du);
         }
     };
+    if constexpr (S == 1) {
+        for (int t = a.T - 1; t >= 0; --t) {
+            load(t, ga, ua);
+            run(t, ga, ua);
+        }
+        return;
+    }
     load(a.T - 1, ga, ua);
     for (int t1 = a.T - 1; t1 >= 0; t1 -= 2 * S) {
         if (t1 - S >= 0) load(t1 - S, gb, ub);
@@ -1520,12 +1534,24 @@ __global__ void __launch_bounds__(256) lif_bwd_kernel(delrec_lif_bwd_args a, Lif
     }
 }
 
+// Blocks of steps loaded ahead pay where the waves in flight leave loads to hide: up to 8 waves to
+// a CU, from 24 steps on forward (the loads past a short run's end are a block's), any number
+// backward; up to 16 waves for long runs. us, one load at a time / blocks, at B N = 131,072 (8
+// waves), 262,144 and 1,048,576:
+//   forward:   T 8 4.3 / 4.8, 5.1 / 8.1, 15.9 / 24.8   T 24 9.7 / 8.8, 13.6 / 15.4, 57.7 / 62.5
+//              T 64 25.6 / 19.4, 31.8 / 38.0, 163 / 165   T 250 176 / 82, 223 / 167, 660 / 614
+//   backward:  T 8 4.6 / 4.0, 5.5 / 5.5, 16.9 / 23.5   T 64 30.5 / 20.4, 35.5 / 35.8, 158 / 187
+//              T 250 168 / 74, 200 / 155, 639 / 649
 void launch_lif(bool fwd, const delrec_lif_fwd_args* fa, const delrec_lif_bwd_args* ba,
-                const Lif& k, hipStream_t stream) {
+                const Lif& k, int cus, hipStream_t stream) {
     const size_t BN = fwd ? (size_t)fa->B * fa->N : (size_t)ba->B * ba->N;
+    const int T = fwd ? fa->T : ba->T;
     const unsigned blocks = (unsigned)((BN + 255) / 256);
-    if (fwd) hipLaunchKernelGGL(lif_fwd_kernel, dim3(blocks), dim3(256), 0, stream, *fa, k);
-    else hipLaunchKernelGGL(lif_bwd_kernel, dim3(blocks), dim3(256), 0, stream, *ba, k);
+    const bool ahead = (BN <= (size_t)512 * cus && (T >= 24 || !fwd)) || (BN <= (size_t)1024 * cus && T >= 100);
+    if (fwd && ahead) hipLaunchKernelGGL(lif_fwd_kernel<kLifFwdSteps>, dim3(blocks), dim3(256), 0, stream, *fa, k);
+    else if (fwd) hipLaunchKernelGGL(lif_fwd_kernel<1>, dim3(blocks), dim3(256), 0, stream, *fa, k);
+    else if (ahead) hipLaunchKernelGGL(lif_bwd_kernel<kLifBwdSteps>, dim3(blocks), dim3(256), 0, stream, *ba, k);
+    else hipLaunchKernelGGL(lif_bwd_kernel<1>, dim3(blocks), dim3(256), 0, stream, *ba, k);
 }
 
 }  // namespace delrec
