@@ -23,6 +23,13 @@ CASES = [
     (40, 8, 10, 'sum', 3.0, True),
     (1, 5, 300, 'mean', None, False),         # more classes than threads
     (1024, 4, 10, 'mean', 2.0, False),        # C5's readout length
+    # around the blocks of sixteen loaded steps
+    (7, 6, 9, 'max', 2.0, False),
+    (8, 6, 9, 'max', 2.0, False),
+    (15, 6, 9, 'max', 2.0, False),
+    (16, 6, 9, 'sum', 2.0, False),
+    (17, 6, 9, 'max', None, False),
+    (31, 6, 9, 'mean', 3.0, True),
 ]
 
 
