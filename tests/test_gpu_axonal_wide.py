@@ -1,9 +1,10 @@
 """Axonal layers past 256 neurons -- the scatter of arriving spikes (``axwide.hip``) and the
 blocked reverse scan without offsets (``hybblock.hip``) -- against the oracle, at their edges:
 one neuron past a wave or a group, two and four neurons per lane, up to 640 and 1,000 neurons
-(the latter's window past the blocked scan's LDS), two, four and eight taps, one, two and four
+(with a window in and past the blocked scan's LDS), two, four and eight taps, one, two and four
 history words, a last partial block of steps, more than 64 arrivals in a step, one step, and the
-neuron's options. Tolerances: ``tests/helpers.py``."""
+neuron's options; and the dense scans, which keep learned spreads, hard taps and more taps (past
+8 forward, 12 backward). Tolerances: ``tests/helpers.py``."""
 
 import ctypes
 
@@ -12,6 +13,7 @@ import torch
 
 from helpers import gen
 from test_gpu_axonal import _check_case
+from test_gpu_modes import test_hard_tap_modes_match_oracle as check_hard_taps
 
 CASES = [
     # T, B, N, dmax, sigma, extra
@@ -26,6 +28,13 @@ CASES = [
     (90, 1, 260, 75.0, 1.0, {'triangle': True}),
     (150, 1, 258, 140.0, 0.0, {'v_reset': -0.2}),
     (1, 2, 300, 5.0, 1.0, {}),
+    (15, 1, 1000, 4.0, 0.5, {'bias': True}),
+    # the dense forward: 11 taps, a spread per source; and the dense backward: 13 taps, a spread
+    (20, 2, 300, 9.0, 4.2, {}),
+    (20, 2, 290, 9.0, 5.5, {'drop': True}),
+    (19, 2, 300, 10.0, 0.7, {'sig_p': True}),
+    (17, 1, 515, 12.0, 3.0, {'sig_p': True, 'bias': True}),
+    (80, 1, 270, 66.0, 0.5, {'sig_p': True}),
 ]
 
 
@@ -33,6 +42,20 @@ CASES = [
 @pytest.mark.parametrize('case', CASES, ids=[f'T{c[0]}N{c[2]}d{c[3]}s{c[4]}{"".join(c[5])}' for c in CASES])
 def test_wide_axonal_matches_oracle(dev, case, monkeypatch):
     _check_case(dev, case, monkeypatch)
+
+
+# the hard-tap forwards (dense) and their straight-through and soft backwards
+HARD = [
+    ('triton_approx', True, 'approx', 20, 2, 300, 12.0, 0.6),
+    ('triton_ste', True, 'ste_round', 20, 2, 290, 9.0, 0.5),
+    ('triton_ste', False, 'ste_interp', 20, 2, 300, 9.0, 1.0),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', HARD, ids=[c[2] for c in HARD])
+def test_wide_axonal_hard_taps_match_oracle(dev, case):
+    check_hard_taps(dev, case)
 
 
 @pytest.mark.gpu

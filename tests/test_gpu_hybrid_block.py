@@ -27,6 +27,8 @@ CASES = [
     (30, 2, 385, (0.0, 28.0), 5, True, 2.5),
     (31, 1, 513, (0.0, 18.0), 3, False, 1.0),
     (22, 1, 600, (0.0, 12.0), 2, True, 0.0),
+    (18, 1, 800, (0.0, 6.0), 3, True, 1.0),
+    (18, 1, 1024, (0.0, 4.0), 2, False, 1.0),       # the limit
     (20, 2, 48, (0.0, 10.0), 3, False, 4.0),        # ten taps
 ]
 

@@ -369,6 +369,9 @@ HYB_G_CASES = [
     (30, 2, 80, (0.0, 14.0), 11, True, 0.0),
     (18, 3, 200, (0.0, 9.0), 5, False, 0.0),
     (20, 2, 128, (0.0, 10.0), 6, True, 0.0, 0, True),
+    # (fp32 weights from N = 176 on take the blocked scan where its ring is of 16 slots)
+    (18, 3, 168, (0.0, 9.0), 5, False, 0.0),
+    (18, 2, 200, (0.0, 9.0), 10, False, 0.0),
 ]
 
 

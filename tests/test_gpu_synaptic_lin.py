@@ -8,6 +8,7 @@ import pytest
 import torch
 
 from helpers import check_grads, first_flip, gen, grad_eps, lif_params, oracle_synaptic, syn_budget
+from test_gpu_synaptic import SYN_CASES, test_synaptic_fwd_bwd_matches_oracle as check_case
 
 CASES = [
     # T, B, N, delays from, to, sigma, options
@@ -76,6 +77,21 @@ def test_interpolated_backward_matches_oracle(dev, case):
     plain = drop is None
     check_grads(got, g64, gref, 2e-2 if bf16 else 1e-4, 1e-5, eps=grad_eps(bf16),
                 budget=syn_budget(g64['x'], y.detach().cpu(), d, sigma, W=W) if plain else None)
+
+
+# the gather per tap, which keeps the spreads per source and the layers whose tables miss LDS, at each
+# of its compiled tap runs (4, 8, 12) and a runtime count; the last two take it without the switch
+GATHER = [SYN_CASES[i] for i in (0, 1, 2, 7, 8)] + [
+    (14, 2, 40, 6.0, 0.3, {'sig_p': True}),
+    (14, 2, 72, 6.0, 4.0, {'sig_p': True, 'bias': True}),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('case', GATHER, ids=[f'N{c[2]}s{c[4]}{"".join(c[5])}' for c in GATHER])
+def test_gather_per_tap_backward_matches_oracle(dev, case, monkeypatch):
+    monkeypatch.setenv('DELREC_SYN_LIN', '0')
+    check_case(dev, case)
 
 
 @pytest.mark.gpu
