@@ -200,7 +200,8 @@ typedef struct {
        below 2. The offset-stacked backward splits the sources by first lag; given these counts
        (e.g. from the forward's own host read) it runs without a host synchronisation,
        otherwise (near_known == 0, as a zeroed struct has it) it reads the first lags back from
-       the device once per call. Counts that do not match the device's make every output NaN. */
+       the device once per call. Counts that do not match the device's make every output NaN
+       there; the scans of a single launch (N <= 1024) only choose their form by near_lt4. */
     int32_t near_known, near_lt4, near_lt2;
 } delrec_syn_bwd_args;
 
@@ -295,7 +296,10 @@ int delrec_axonal_bwd(const delrec_axonal_bwd_args* a, void* stream);
  * a->workspace / workspace_bytes are ignored. Scratch is a 64 MiB array of the library's own
  * device memory, one per GPU, held until the process ends (looked up on the first call on a
  * device); sizes whose workspace (delrec_query_workspace, DELREC_WS_AXONAL_BWD) exceeds it
- * return DELREC_ERR_SCRATCH. Calls on one GPU share that array: calls that overlap on one
+ * return DELREC_ERR_SCRATCH -- past 256 neurons, the workspace without the blocked scan's
+ * operands, that is a second (T,B,N) buffer, the packed W and 2 N + 1 ints at its end: where
+ * the array does not hold these too (N = 512, B = 32: from about T = 375 on), the call runs in
+ * the dense scan, about five times slower. Calls on one GPU share that array: calls that overlap on one
  * GPU (other streams, other threads) race and must not be issued. Allocates nothing. */
 int delrec_axonal_bwd_noalloc(const delrec_axonal_bwd_args* a, void* stream);
 int delrec_syn_fwd(const delrec_syn_fwd_args* a, void* stream);

@@ -435,8 +435,7 @@ void syn_fwd_ws(C& c, int T, int B, int N, int L, bool hybrid, bool bf16, int ta
 }
 
 // The blocked hybrid backward (hybblock.hip): N <= 1024 with the offsets' range known, unless a
-// switch asks for another form. `early`: how many steps before the first possible lag 1 the
-// earliest tap of positive weight may start (0 where every lag is >= 1).
+// switch asks for another form.
 bool hyb_block_on(int N, bool hybrid, int offc) {
     const char* hs = getenv("DELREC_SYN_HYBSTEP");
     const char* ls = getenv("DELREC_SYN_LAGSTEP");
@@ -444,8 +443,9 @@ bool hyb_block_on(int N, bool hybrid, int offc) {
            getenv_flag_off("DELREC_SYN_BWD_HYB") && !(hs && hs[0] == '1') && !(ls && ls[0] == '1');
 }
 
-// the longest early run for a smallest delay (rounded up to the compiled 1, 2, 4, 8; a little
-// slack, so that the device's own fp32 first lag is never below it); 16: longer than compiled
+// The slots of a near sum for a smallest delay: one, and one more for each step that the earliest tap
+// of positive weight starts before lag 1; rounded up to the compiled 1, 2, 4, 8, with a little
+// slack, so that the device's own fp32 first lag is never below it. 16: longer than compiled.
 int hyb_block_early(float d_min, float s, bool lags_ok) {
     if (lags_ok) return 1;
     const double lo = std::floor(1.0 + (double)d_min - (double)s - 1e-3) + 1.0;

@@ -18,15 +18,20 @@
 //     G(t - 1), .. over the connections whose lag is still >= 1 -- the slots of the steps not
 //     yet formed hold 0, so these are the same run of slots, started earlier.
 //
-// Bound: the LDS reads of gr (4 bytes per connection and step at 128 B/clk: 2,048 clk a step at
-// N = 256, 8,192 at N = 512; without offsets one read serves 16 receivers' multiply-adds, whose
-// issue, 4,096 clk at N = 512, is the bound then) and the two exchanges of a step.
-// Measured (scan): T250 B128 N256 sigma 1, 5 offsets, fp32 W 0.65 ms, 2.6 us a step (23.5 ms with
-// the per-tap gather of syn_bwd_kernel); T256 B256 N512 sigma 0, 9 offsets, bf16 W 1.8 ms (2.22 ms
-// with syn_bwd_hyb_g); axonal T250 B256 N512 sigma 1 fp32 W 1.6 ms (8.70 ms with the dense
-// product streamed per step, axonal_bwd_kernel). A group's whole block taken in one step by its
-// own wave alone: 5.2 ms at N = 512 (one wave per SIMD at a time hides nothing); neurons on the
-// summing waves instead of waves of their own: 2.0 ms (their registers together spill).
+// Bound: the multiply-adds' issue (with offsets: one, an address and a share of the decode for each
+// connection of a block), then the LDS reads of gr (4 bytes per connection and step at 128 B/clk)
+// and the two exchanges of a step. Share of the kernel's clocks, from counters:
+//   T256 B256 N512 sigma 0, 9 offsets, bf16 W: vector issue 83 %, LDS 58 % (1 % of it conflicts)
+//   T250 B128 N256 sigma 1, 5 offsets, fp32 W: vector issue 68 %, LDS 47 % (4 % conflicts)
+//   axonal T250 B256 N512 sigma 1, fp32 W: vector issue 64 %, LDS 20 % (one read serves 16
+//     receivers' multiply-adds), operands from L2 30 B/clk a CU
+// Measured (scan): those three 1.7 ms (2.2 ms with syn_bwd_hyb_g), 0.65 ms, 2.6 us a step (23.5 ms
+// with the gather per tap, syn_bwd_kernel) and 1.56 ms (8.70 ms with the dense product streamed per
+// step, axonal_bwd_kernel). A group's whole block taken in one step by its own wave alone: 5.2
+// ms at N = 512 (one wave per SIMD at a time hides nothing); neurons on the summing waves instead
+// of waves of their own: 2.0 ms. Registers (of 128): runs of 1 and 2 slots spill up to 8; of 4 37
+// to 46, and of 8 137 to 154, with four neurons a lane; scalar ones spill to lanes of vector
+// registers (48 to 80 bytes of scratch a lane).
 #include <algorithm>
 
 #include "common.h"
@@ -165,7 +170,7 @@ __global__ void __launch_bounds__(256) hyb_block_pack_kernel(HybBlk p, uint4* wq
 // slots never wraps. NT slots per near sum, t + 2 - NT .. t + 1. Near and far operands have
 // their own registers, filled from L2 in chunks of 16 receivers, each register refilled with the
 // following chunk's as soon as it is used.
-// The first waves of a workgroup (p.nwg of them, up to 12) do the sums, the others (up to 4) run
+// The first waves of a workgroup (p.nwg of them, 4 to 14) do the sums, the others (1 to 4) run
 // NPL neurons per lane: roles of their own, so that neither holds the other's registers. A step:
 // near sums | barrier | far sums, beside the neurons | barrier.
 template <int GPW, int NPL, bool WBF, bool OFF, int R, int PITCH, int NT>
@@ -651,7 +656,7 @@ HybBlkShape hyb_block_shape(int N, int L, bool bf16, bool offsets, int D, int KF
     q.NPL = N <= 192 ? 1 : N <= 384 ? 2 : 4;
     q.NCl = (N + 63) / 64;
     const int neuron_waves = (N + 64 * q.NPL - 1) / (64 * q.NPL);
-    q.nwg = std::min(16 - neuron_waves, std::max(groups * std::min(q.NCl, 4), 4));   // far groups per wave: at most 1, 2, 2, 3, 6
+    q.nwg = std::min(16 - neuron_waves, std::max(groups * std::min(q.NCl, 4), 4));   // far groups per wave: at most 1, 2, 3, 6 (N <= 192, 384, 512, 1024)
     q.block = (q.nwg + neuron_waves) * 64;
     q.Ns = groups * 16;
     q.RG = std::max(L, 8) + 1;                             // steps t + 1 .. t + L - 1, blocks to t + 7

@@ -14,8 +14,10 @@
 // A connection is 8 bytes: W in fp32 and (n mod R as a byte offset) << 24 | f in 23 bits, read as
 // the float 1 + f (the pair holds A - D). Lanes are sources, a wave reads one receiver row at a
 // time: distinct slots are distinct banks, equal ones broadcast.
-// Bound: the operands' bytes from L2 (524 KB a step at N = 256, 64 B/clk per CU), then the pair
-// reads (8 bytes at 128 B/clk).
+// Bound: LDS, 85 % of the kernel's clocks at T250 B256 N256 sigma 1, two thirds of that conflicts (the
+// pairs of a wave's lanes, and the neurons' own rows, which all start in one bank); then the
+// operands from L2 (524 KB a step, 36 of 64 B/clk per CU) and vector issue (43 %). Where s is no whole
+// number the kernel spills 23 registers of 128.
 // Measured (scan), with the taps walked one by one (syn_bwd_kernel) / with the tables:
 //   T250 B256 N256 sigma 1 8.51 / 1.64 ms (34 / 6.6 us a step); T48 B64: N 100 sigma 1 0.74 / 0.11,
 //   N 160 sigma 0.4 0.73 / 0.29, N 256 sigma 3 2.16 / 0.38, N 512 sigma 0 2.47 / 0.84 ms.
